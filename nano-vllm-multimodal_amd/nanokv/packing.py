@@ -17,6 +17,7 @@ The result is a :class:`Context` with the fields of the reference's
 from __future__ import annotations
 
 import ctypes
+import gc
 from dataclasses import dataclass
 from typing import Iterable, Sequence
 
@@ -152,6 +153,11 @@ class DecodeGraphBuffers:
             raise ValueError("max_num_seqs and max_blocks must be positive")
         if max_num_seqs > _lib.NKV_MAX_PACK_SEQS:
             raise ValueError(f"at most {_lib.NKV_MAX_PACK_SEQS} sequences per decode graph")
+        # A capture follows.  PyTorch-ROCm's CUDAGraph destructor synchronises
+        # the device, which is an error while a stream captures and ends the
+        # process: a graph that only a reference cycle still holds is freed
+        # now, not by a garbage collection in the middle of the capture.
+        gc.collect()
         device = torch.device(device)
         zeros = lambda *shape: torch.zeros(shape, dtype=torch.int32, device=device)  # noqa: E731
         return cls(zeros(max_num_seqs), zeros(max_num_seqs), zeros(max_num_seqs, max_blocks),

@@ -106,3 +106,22 @@ def test_index_validation_flag_is_read_per_call(host):
 
 def test_build_id_matches_the_sources_and_torch(host):
     assert host.build_id() == nkv_build.host_build_id()
+
+
+def test_graph_buffers_collect_dead_cycles_before_a_capture():
+    """Allocating a decode graph's buffers frees what only reference cycles
+    hold (a dead CUDAGraph collected during the capture that follows would
+    end the process)."""
+    import weakref
+
+    from nanokv.packing import DecodeGraphBuffers
+
+    class Holder:
+        pass
+
+    holder = Holder()
+    holder.self = holder
+    dead = weakref.ref(holder)
+    del holder
+    DecodeGraphBuffers.allocate("cpu", 2, 3)
+    assert dead() is None
