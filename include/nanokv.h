@@ -413,7 +413,7 @@ int nkv_paged_attention_decode(const void* q, int64_t q_seq_stride,
  *
  * nkv_build_prefill_plan cuts every request's queries into tiles of
  *   nkv_prefill_tile_tokens(G) tokens (128 / G) and writes one int4
- *   {seq, token0, tokens, 0} per tile into `plan` (capacity >=
+ *   {seq, token0, tokens, key tiles seen} per tile into `plan` (capacity >=
  *   nkv_prefill_plan_capacity(total query tokens, num_seqs, G)).  Tiles
  *   are listed by the number of keys they see, most first (plans of up to
  *   2048 entries; longer ones request by request, last tile first).  It
@@ -425,6 +425,12 @@ int nkv_paged_attention_decode(const void* q, int64_t q_seq_stride,
  *   out are [total query tokens, num_q_heads, head_dim] with token strides
  *   q_token_stride / out_token_stride elements (q rows 16-byte aligned,
  *   out rows 8-byte aligned).  Needs no workspace.
+ * nkv_paged_attention_prefill_split is the same call with a workspace of
+ *   nkv_prefill_workspace_bytes(capacity, num_kv_heads, table_stride *
+ *   block_size) bytes (16-byte aligned): a launch too short to fill the chip
+ *   then cuts the keys of its tiles into pieces, one workgroup each, and
+ *   merges their fp32 partials.
+ *   Where that size is 0, or with a null workspace, it cuts nothing.
  */
 int64_t nkv_prefill_tile_tokens(int64_t group);
 int64_t nkv_prefill_plan_capacity(int64_t total_q_tokens, int64_t num_seqs,
@@ -443,6 +449,17 @@ int nkv_paged_attention_prefill(const void* q, int64_t q_token_stride,
                                 int64_t head_dim, int64_t block_size,
                                 int64_t num_blocks, float scale, int32_t dtype,
                                 void* out, int64_t out_token_stride, void* stream);
+int64_t nkv_prefill_workspace_bytes(int64_t capacity, int64_t num_kv_heads,
+                                    int64_t max_keys);
+int nkv_paged_attention_prefill_split(
+    const void* q, int64_t q_token_stride, const void* key_cache,
+    const void* value_cache, const int32_t* block_tables, int64_t table_stride,
+    const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, const void* plan,
+    int64_t capacity, int64_t num_seqs, int64_t num_kv_heads,
+    int64_t num_q_heads, int64_t head_dim, int64_t block_size,
+    int64_t num_blocks, float scale, int32_t dtype, void* out,
+    int64_t out_token_stride, void* workspace, int64_t workspace_bytes,
+    void* stream);
 
 /*
  * Host-to-device transfer lane: a non-blocking transfer stream (default

@@ -30,6 +30,7 @@
 //   * the query tiles of one kv head run on one XCD (shared L2).
 // Invalid block ids (outside [0, num_blocks), or past the table) drop their
 // keys, as in the decode kernel.
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
@@ -65,8 +66,9 @@ constexpr float kRescaleLog2 = 8.f;
 // being read from the one being copied into.
 constexpr int kTileChunks = kPfKeys * 16;  // 16-byte chunks per K or V tile
 
-// Plan: one int4 {seq, token0, tokens, 0} per workgroup: tokens [token0,
-// token0 + tokens) of sequence seq's queries, tokens <= tile_tokens.
+// Plan: one int4 {seq, token0, tokens, key_tiles} per query tile: tokens
+// [token0, token0 + tokens) of sequence seq's queries, tokens <=
+// tile_tokens, and the number of 64-key tiles they see.
 // Entries past the total get tokens = 0.  The tiles are listed longest
 // first (most visible keys: the keys of a tile's last query), so that the
 // longest workgroups start first and the short ones fill the tail; ties in
@@ -102,7 +104,9 @@ __global__ __launch_bounds__(kPfPlanThreads) void prefill_plan_kernel(
     const int32_t tiles = s_first[i + 1] - s_first[i];
     const int32_t t0 = (tiles - 1 - (e - s_first[i])) * tile_tokens;
     const int32_t len = cu_seqlens_q[i + 1] - cu_seqlens_q[i];
-    return make_int4(i, t0, min(tile_tokens, len - t0), 0);
+    const int32_t ntok = min(tile_tokens, len - t0);
+    const int32_t visible = max(0, cu_seqlens_k[i + 1] - cu_seqlens_k[i] - len + t0 + ntok);
+    return make_int4(i, t0, ntok, visible / kPfKeys + (visible % kPfKeys != 0 ? 1 : 0));
   };
   if (sort && total <= kPfSortMax) {  // one workgroup (the launch makes sure)
     // Sort keys: (2^31 - 1 - visible keys) << 32 | e, ascending; padding last.
@@ -247,7 +251,225 @@ __device__ __forceinline__ TileId tile_of(uint32_t id, int32_t num_kv_heads, int
   return TileId{static_cast<int32_t>(id / num_kv_heads), static_cast<int32_t>(id % num_kv_heads)};
 }
 
-template <int G, bool kWide, bool kHalf>
+// The key split.  A workgroup walks the keys of its query tile one 64-key
+// tile after another (about 1.3 us each), so a launch of few query tiles
+// lasts as long as its longest one while most of the chip idles: 4 requests
+// of ~98 new tokens over 6k-12k cached ones are 64 workgroups (8 kv heads)
+// and took 262 us, 195 key tiles in a row on a quarter of the CUs.  Such a
+// launch cuts each tile's keys into pieces of at most C key tiles, one
+// workgroup each, whose fp32 partials (max, weight sum, output sums) a merge
+// kernel adds up: that case went to 56-62 us, one 40-token chunk over 14k
+// cached rows from 311 to 38 us.
+// One kv head can have slots = 512 / Hkv workgroups resident at once (two
+// per CU).  With T key tiles in the whole plan, C = T / (slots - tiles)
+// makes at most T / C + tiles <= slots pieces, which start together; more
+// would leave a second, nearly empty round (with C = T / slots, 284
+// workgroups of 2 kv heads lost 5% instead).  A piece of fewer than
+// kSplitMinTiles key tiles costs more to start and merge than it saves (2,
+// 4 and 6 measure alike).
+#ifndef NKV_PF_SPLIT_MIN_TILES
+#define NKV_PF_SPLIT_MIN_TILES 4  // shortest piece, in key tiles
+#endif
+#ifndef NKV_PF_SPLIT_MIN_SEEN
+#define NKV_PF_SPLIT_MIN_SEEN 8  // key tiles some query tile must be able to see
+#endif
+constexpr int kSplitMinTiles = NKV_PF_SPLIT_MIN_TILES;
+constexpr int kSplitMinSeen = NKV_PF_SPLIT_MIN_SEEN;
+constexpr int kSplitSlots = 256 * kPfBlocksPerCU;  // workgroups resident on the chip
+constexpr int kSplitMaxTiles = kSplitSlots;        // plan entries find_piece scans
+constexpr int kSplitPerLane = kSplitMaxTiles / kWave;
+constexpr int kSplitTileClamp = 1 << 20;  // key tiles of one query tile, as counted: sums fit 31 bits
+
+__host__ __device__ constexpr int32_t split_slots(int64_t num_kv_heads) {
+  return num_kv_heads < kSplitSlots ? static_cast<int32_t>(kSplitSlots / num_kv_heads) : 1;
+}
+// Whether a launch of this many plan entries cuts its keys, no request
+// having more than max_keys of them: when it is one round of workgroups (cut
+// launches of two rounds and more lost 10-20%: 868 workgroups of 4 kv heads
+// took 80 us against 64) and some tile may see enough keys to pay for the
+// merge launch (about 4 us, three key tiles; 456 workgroups over at most 4
+// key tiles lost 7%).
+constexpr bool uses_split(int64_t capacity, int64_t num_kv_heads, int64_t max_keys) {
+  return num_kv_heads <= kSplitSlots && capacity * num_kv_heads <= kSplitSlots &&
+         max_keys > int64_t{kSplitMinSeen} * kPfKeys;
+}
+// Pieces of one kv head: those of at most slots - 1 cut tiles and the whole
+// tiles, T / C + tiles <= slots in all (C >= T when every slot has a tile).
+constexpr int64_t split_pieces(int64_t num_kv_heads) { return split_slots(num_kv_heads) + 1; }
+// Partials of one kv head: no more than its pieces.
+constexpr int64_t split_partials(int64_t num_kv_heads) { return split_pieces(num_kv_heads); }
+// One partial: 128 x 128 output sums in the order the merge reads them
+// (16-row block, 16-dim block, lane: 1 KiB per wavefront access), then each
+// row's (max, weight sum).
+constexpr int64_t kPartSums = int64_t{kPfRows} * kPfDim;
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+
+struct Piece {
+  int32_t entry;     // plan entry, -1: no such piece
+  int32_t piece;     // which of its pieces
+  int32_t pieces;    // how many it has
+  int32_t partial;   // its partial's index (of its kv head); meaningful when pieces > 1
+};
+
+// Piece `want` of the plan's pieces, entry after entry.  Every wavefront
+// finds it for itself (no barrier): a lane counts up to kSplitPerLane
+// consecutive entries, then scans across the lanes.
+__device__ __forceinline__ Piece find_piece(const int4* __restrict__ plan, int32_t capacity,
+                                            int32_t want, int32_t slots, int lane) {
+  const int32_t per = (capacity + kWave - 1) / kWave;
+  int32_t count[kSplitPerLane];  // key tiles, then pieces, of the lane's entries
+  int32_t key_tiles = 0, tiles = 0;
+#pragma unroll
+  for (int i = 0; i < kSplitPerLane; ++i) {
+    count[i] = 0;
+    if (i < per && lane * per + i < capacity) {
+      const int4 e = plan[lane * per + i];
+      if (e.z > 0 && e.w > 0) count[i] = min(e.w, kSplitTileClamp);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kSplitPerLane; ++i) {
+    key_tiles += count[i];
+    tiles += count[i] > 0 ? 1 : 0;
+  }
+#pragma unroll
+  for (int d = kWave / 2; d > 0; d >>= 1) {
+    key_tiles += __shfl_xor(key_tiles, d, kWave);
+    tiles += __shfl_xor(tiles, d, kWave);
+  }
+  const int32_t budget = max(1, slots - tiles);
+  const int32_t size = max(kSplitMinTiles, (key_tiles + budget - 1) / budget);
+  // Pieces in the low half, partials in the high half: both below 2^15.
+  int32_t mine = 0;
+#pragma unroll
+  for (int i = 0; i < kSplitPerLane; ++i) {
+    if (i < per) {
+      count[i] = (count[i] + size - 1) / size;
+      mine += count[i] > 1 ? count[i] * 0x10001 : count[i];
+    }
+  }
+  const int32_t upto = wave_inclusive_scan(mine);
+  const uint64_t past = __ballot((upto & 0xFFFF) > want);
+  if (past == 0) return Piece{-1, 0, 0, 0};
+  const int owner = __builtin_ctzll(past);
+  const int32_t before = upto - mine;
+  int32_t left = want - (before & 0xFFFF);  // in the owner lane: pieces of its entries before it
+  int32_t partial = before >> 16;
+  Piece out{-1, 0, 0, 0};
+#pragma unroll
+  for (int i = 0; i < kSplitPerLane; ++i) {
+    if (i < per && out.entry < 0) {
+      if (left < count[i]) {
+        out = Piece{lane * per + i, left, count[i], partial + left};
+      } else {
+        left -= count[i];
+        partial += count[i] > 1 ? count[i] : 0;
+      }
+    }
+  }
+  return Piece{__builtin_amdgcn_readlane(out.entry, owner), __builtin_amdgcn_readlane(out.piece, owner),
+               __builtin_amdgcn_readlane(out.pieces, owner),
+               __builtin_amdgcn_readlane(out.partial, owner)};
+}
+
+// Adds the partials of the tiles that were cut.  A wavefront merges 16 rows
+// x 64 dims of one (tile, kv head); a lane holds the same row and dims as in
+// the attention kernel, so the row's weights need no exchange and every
+// access is 1 KiB.  Four pieces are in flight at once.
+constexpr int kMergeBatch = 4;
+constexpr int kMergeWaves = 4;
+constexpr int kMergeUnits = kPfRows / 16 * 2;  // wavefronts per (tile, kv head)
+static_assert(kMergeUnits % kMergeWaves == 0, "whole workgroups per tile");
+
+template <bool kHalf>
+__global__ __launch_bounds__(kMergeWaves* kWave) void prefill_merge_kernel(
+    const float* __restrict__ part_acc, const f32x2* __restrict__ part_ml,
+    const int2* __restrict__ tile_parts, const int4* __restrict__ plan, int32_t num_seqs,
+    const int32_t* __restrict__ cu_seqlens_q, const int32_t* __restrict__ cu_seqlens_k,
+    int32_t num_kv_heads, int32_t group, uint16_t* __restrict__ out, int64_t out_token_stride) {
+  typedef typename Elem<kHalf>::T T;
+  typedef typename Elem<kHalf>::X4 X4;
+  constexpr int kBlocksPerTile = kMergeUnits / kMergeWaves;
+  const int32_t tile = static_cast<int32_t>(blockIdx.x) / kBlocksPerTile;
+  const int32_t e = tile / num_kv_heads;
+  const int32_t kh = tile % num_kv_heads;
+  // The attention kernel's checks: it wrote nothing for these entries.
+  const int4 entry = plan[e];
+  const int32_t seq = entry.x;
+  const int32_t tok0 = entry.y;
+  const int32_t ntok = entry.z;
+  if (ntok <= 0 || entry.w <= 0 || ntok > kPfRows / group || seq < 0 || seq >= num_seqs || tok0 < 0) return;
+  const int2 parts = tile_parts[e];  // {first partial, pieces}
+  const int32_t q_begin = cu_seqlens_q[seq];
+  const int32_t lq = cu_seqlens_q[seq + 1] - q_begin;
+  const int32_t lk = cu_seqlens_k[seq + 1] - cu_seqlens_k[seq];
+  if (parts.y <= 1 || lk < lq || tok0 + ntok > lq) return;
+
+  const int lane = threadIdx.x & (kWave - 1);
+  const int unit = static_cast<int>(blockIdx.x) % kBlocksPerTile * kMergeWaves +
+                   __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int block = unit >> 1;       // 16-row block
+  const int db0 = (unit & 1) * 4;    // first 16-dim block
+  const int m = block * 16 + (lane & 15);
+  float run_max = -INFINITY, run_sum = 0.f;
+  f32x4 acc[4];
+#pragma unroll
+  for (int d = 0; d < 4; ++d) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int32_t p = 0; p < parts.y; p += kMergeBatch) {
+    f32x2 ml[kMergeBatch];
+    f32x4 v[kMergeBatch][4];
+#pragma unroll
+    for (int i = 0; i < kMergeBatch; ++i) {
+      const int64_t slot =
+          static_cast<int64_t>(parts.x + min(p + i, parts.y - 1)) * num_kv_heads + kh;
+      ml[i] = part_ml[slot * kPfRows + m];
+      const f32x4* src = reinterpret_cast<const f32x4*>(part_acc + slot * kPartSums) +
+                         (block * 8 + db0) * kWave + lane;
+#pragma unroll
+      for (int d = 0; d < 4; ++d) v[i][d] = src[d * kWave];
+    }
+    float top = run_max;
+#pragma unroll
+    for (int i = 0; i < kMergeBatch; ++i) {
+      if (p + i >= parts.y) ml[i] = f32x2{-INFINITY, 0.f};  // a repeat of the last piece
+      top = fmaxf(top, ml[i].x);
+    }
+    const float keep = run_max == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(run_max - top);
+    run_sum *= keep;
+#pragma unroll
+    for (int d = 0; d < 4; ++d) acc[d] *= keep;
+#pragma unroll
+    for (int i = 0; i < kMergeBatch; ++i) {
+      // A piece without visible keys has max -inf and sum 0 (and, with no
+      // key tile at all, unwritten sums).  Max -inf with another sum means
+      // NaN scores: the NaN goes on.
+      if (ml[i].x == -INFINITY && ml[i].y == 0.f) continue;
+      const float f = ml[i].x == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(ml[i].x - top);
+      run_sum = __builtin_fmaf(ml[i].y, f, run_sum);
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[d][j] = __builtin_fmaf(v[i][d][j], f, acc[d][j]);
+      }
+    }
+    run_max = top;
+  }
+  const int t = m / group;
+  if (t >= ntok) return;
+  const float inv = run_sum > 0.f ? 1.f / run_sum : 0.f;
+  uint16_t* orow = out + static_cast<int64_t>(q_begin + tok0 + t) * out_token_stride +
+                   (kh * group + m % group) * kPfDim + 16 * db0 + 4 * (lane >> 4);
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const X4 w = {static_cast<T>(acc[d].x * inv), static_cast<T>(acc[d].y * inv),
+                  static_cast<T>(acc[d].z * inv), static_cast<T>(acc[d].w * inv)};
+    *reinterpret_cast<X4*>(orow + 16 * d) = w;
+  }
+}
+
+// kSplit: one workgroup per piece and kv head, max_pieces pieces per kv head
+// in the grid; otherwise one per plan entry and kv head (no workspace).
+template <int G, bool kWide, bool kHalf, bool kSplit>
 __global__ __launch_bounds__(kPfThreads, kPfBlocksPerCU) void attn_prefill_kernel(
     const uint16_t* __restrict__ q, int64_t q_token_stride,
     const uint8_t* __restrict__ key_cache, const uint8_t* __restrict__ value_cache,
@@ -255,7 +477,8 @@ __global__ __launch_bounds__(kPfThreads, kPfBlocksPerCU) void attn_prefill_kerne
     int32_t block_shift, int32_t num_blocks, int32_t num_kv_heads,
     const int32_t* __restrict__ cu_seqlens_q, const int32_t* __restrict__ cu_seqlens_k,
     const int4* __restrict__ plan, int32_t capacity, int32_t xcd_layout, int32_t num_seqs,
-    float scale_log2, uint16_t* __restrict__ out, int64_t out_token_stride) {
+    float scale_log2, uint16_t* __restrict__ out, int64_t out_token_stride, int32_t max_pieces,
+    float* __restrict__ part_acc, f32x2* __restrict__ part_ml, int2* __restrict__ tile_parts) {
   constexpr int kTileTokens = kPfRows / G;
   typedef Elem<kHalf> E;
   typedef typename E::T T;
@@ -268,7 +491,17 @@ __global__ __launch_bounds__(kPfThreads, kPfBlocksPerCU) void attn_prefill_kerne
   __shared__ int32_t rows_buf[4][kPfKeys];  // physical row of each key of a tile, -1 if invalid
   __shared__ int32_t invalid_buf[4];        // whether a tile has an invalid row
 
-  const TileId id = tile_of(blockIdx.x, num_kv_heads, capacity, xcd_layout);
+  TileId id = tile_of(blockIdx.x, num_kv_heads, kSplit ? max_pieces : capacity, xcd_layout);
+  Piece part{id.entry, 0, 1, 0};
+  if constexpr (kSplit) {
+    if (id.entry >= max_pieces) return;
+    part = find_piece(plan, capacity, id.entry, split_slots(num_kv_heads), threadIdx.x % kWave);
+    id.entry = part.entry;
+    if (part.entry < 0) return;
+    if (part.piece == 0 && id.kv_head == 0 && threadIdx.x == 0) {
+      tile_parts[part.entry] = make_int2(part.partial, part.pieces);
+    }
+  }
   if (id.entry >= capacity) return;
   const int4 entry = plan[id.entry];
   const int32_t seq = entry.x;
@@ -315,7 +548,21 @@ __global__ __launch_bounds__(kPfThreads, kPfBlocksPerCU) void attn_prefill_kerne
     }
   }
 
-  const int32_t num_tiles = (num_keys + kPfKeys - 1) / kPfKeys;
+  // The piece's key tiles [tile_begin, tile_begin + num_tiles) of all the
+  // tile sees; the loop counts from 0.
+  const int32_t all_tiles = (num_keys + kPfKeys - 1) / kPfKeys;
+  int32_t key_begin = 0, num_tiles = all_tiles;
+  const int64_t part_slot = static_cast<int64_t>(part.partial) * num_kv_heads + kh;
+  if constexpr (kSplit) {
+    const int64_t tiles64 = all_tiles;
+    const int32_t tile_begin = static_cast<int32_t>(tiles64 * part.piece / part.pieces);
+    num_tiles = static_cast<int32_t>(tiles64 * (part.piece + 1) / part.pieces) - tile_begin;
+    key_begin = tile_begin * kPfKeys;
+    if (num_tiles <= 0) {  // more pieces than key tiles (a plan for other lengths)
+      if (part.pieces > 1 && tid < kPfRows) part_ml[part_slot * kPfRows + tid] = f32x2{-INFINITY, 0.f};
+      return;
+    }
+  }
   float row_max[2] = {-INFINITY, -INFINITY};
   // O^T blocks: dims 16 * db + 4 * g4 + i of row m.  Block 8 multiplies P
   // by a row of ones (dim 128 of an extended V^T), so its first dim holds
@@ -341,12 +588,12 @@ __global__ __launch_bounds__(kPfThreads, kPfBlocksPerCU) void attn_prefill_kerne
     // for one round trip through the table, not one per tile.
     int32_t first_blocks[3];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) first_blocks[i] = i < num_tiles ? map.block_of(i * kPfKeys + lane) : -1;
-    if (num_tiles > 3) ahead_block = map.block_of(3 * kPfKeys + lane);
+    for (int i = 0; i < 3; ++i) first_blocks[i] = i < num_tiles ? map.block_of(key_begin + i * kPfKeys + lane) : -1;
+    if (num_tiles > 3) ahead_block = map.block_of(key_begin + 3 * kPfKeys + lane);
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
       if (i < num_tiles) {
-        resolve_rows(rows_buf[i], &invalid_buf[i], map, i * kPfKeys, first_blocks[i], lane);
+        resolve_rows(rows_buf[i], &invalid_buf[i], map, key_begin + i * kPfKeys, first_blocks[i], lane);
       }
     }
   }
@@ -382,7 +629,7 @@ __global__ __launch_bounds__(kPfThreads, kPfBlocksPerCU) void attn_prefill_kerne
     u32x4* const k_next = kCur == 0 ? k_buf1 : k_buf0;  // K(tile + 1)
     u32x4* const v_cur = kCur == 0 ? v_buf0 : v_buf1;
     u32x4* const v_next = kCur == 0 ? v_buf1 : v_buf0;
-    const int32_t key0 = tile * kPfKeys;
+    const int32_t key0 = key_begin + tile * kPfKeys;
     const int slot = tile & 3;
     __builtin_amdgcn_s_waitcnt(0);  // this wavefront's copies of K(tile + 1), V(tile) have landed
     __syncthreads();                // ... and everyone's; tile - 1 is consumed
@@ -520,6 +767,14 @@ __global__ __launch_bounds__(kPfThreads, kPfBlocksPerCU) void attn_prefill_kerne
     const float total = row4_sum(g4 == 0 ? acc[8][mb][0] : 0.f);
     const int m = wave * 32 + mb * 16 + c16;
     const int t = m / G;
+    if (kSplit && part.pieces > 1) {  // this piece's partial, padding rows included (the merge skips them)
+      const int block = wave * 2 + mb;
+      if (g4 == 0) part_ml[part_slot * kPfRows + block * 16 + c16] = f32x2{row_max[mb], total};
+      f32x4* dst = reinterpret_cast<f32x4*>(part_acc + part_slot * kPartSums) + block * 8 * kWave + lane;
+#pragma unroll
+      for (int db = 0; db < 8; ++db) dst[db * kWave] = acc[db][mb];
+      continue;
+    }
     if (t >= ntok) continue;
     const float inv = total > 0.f ? 1.f / total : 0.f;
     uint16_t* orow = out + static_cast<int64_t>(q_begin + tok0 + t) * out_token_stride +
@@ -537,21 +792,26 @@ __global__ __launch_bounds__(kPfThreads, kPfBlocksPerCU) void attn_prefill_kerne
 using PrefillKernel = void (*)(const uint16_t*, int64_t, const uint8_t*, const uint8_t*,
                                const int32_t*, int64_t, int32_t, int32_t, int32_t, int32_t,
                                const int32_t*, const int32_t*, const int4*, int32_t, int32_t,
-                               int32_t, float, uint16_t*, int64_t);
+                               int32_t, float, uint16_t*, int64_t, int32_t, float*, f32x2*, int2*);
 
-template <bool kWide, bool kHalf>
+template <bool kWide, bool kHalf, bool kSplit>
 PrefillKernel prefill_kernel_for(int64_t group) {
   switch (group) {
-    case 1: return attn_prefill_kernel<1, kWide, kHalf>;
-    case 2: return attn_prefill_kernel<2, kWide, kHalf>;
-    case 3: return attn_prefill_kernel<3, kWide, kHalf>;
-    case 4: return attn_prefill_kernel<4, kWide, kHalf>;
-    case 5: return attn_prefill_kernel<5, kWide, kHalf>;
-    case 6: return attn_prefill_kernel<6, kWide, kHalf>;
-    case 7: return attn_prefill_kernel<7, kWide, kHalf>;
-    case 8: return attn_prefill_kernel<8, kWide, kHalf>;
+    case 1: return attn_prefill_kernel<1, kWide, kHalf, kSplit>;
+    case 2: return attn_prefill_kernel<2, kWide, kHalf, kSplit>;
+    case 3: return attn_prefill_kernel<3, kWide, kHalf, kSplit>;
+    case 4: return attn_prefill_kernel<4, kWide, kHalf, kSplit>;
+    case 5: return attn_prefill_kernel<5, kWide, kHalf, kSplit>;
+    case 6: return attn_prefill_kernel<6, kWide, kHalf, kSplit>;
+    case 7: return attn_prefill_kernel<7, kWide, kHalf, kSplit>;
+    case 8: return attn_prefill_kernel<8, kWide, kHalf, kSplit>;
     default: return nullptr;
   }
+}
+template <bool kWide>
+PrefillKernel prefill_kernel_for(int64_t group, bool half, bool split) {
+  if (half) return split ? prefill_kernel_for<kWide, true, true>(group) : prefill_kernel_for<kWide, true, false>(group);
+  return split ? prefill_kernel_for<kWide, false, true>(group) : prefill_kernel_for<kWide, false, false>(group);
 }
 
 }  // namespace
@@ -606,6 +866,17 @@ extern "C" int nkv_build_prefill_plan(const int32_t* cu_seqlens_q, const int32_t
   return nkv_check_launch("nkv_build_prefill_plan");
 }
 
+extern "C" int64_t nkv_prefill_workspace_bytes(int64_t capacity, int64_t num_kv_heads,
+                                               int64_t max_keys) {
+  using namespace nkv;
+  if (capacity <= 0 || num_kv_heads <= 0 || capacity > INT32_MAX ||
+      !uses_split(capacity, num_kv_heads, max_keys)) {
+    return 0;
+  }
+  const int64_t partials = split_partials(num_kv_heads) * num_kv_heads;
+  return partials * (kPartSums * 4 + kPfRows * 8) + capacity * 8;
+}
+
 extern "C" int nkv_paged_attention_prefill(
     const void* q, int64_t q_token_stride, const void* key_cache, const void* value_cache,
     const int32_t* block_tables, int64_t table_stride, const int32_t* cu_seqlens_q,
@@ -613,6 +884,19 @@ extern "C" int nkv_paged_attention_prefill(
     int64_t num_kv_heads, int64_t num_q_heads, int64_t head_dim, int64_t block_size,
     int64_t num_blocks, float scale, int32_t dtype, void* out, int64_t out_token_stride,
     void* stream) {
+  return nkv_paged_attention_prefill_split(
+      q, q_token_stride, key_cache, value_cache, block_tables, table_stride, cu_seqlens_q,
+      cu_seqlens_k, plan, capacity, num_seqs, num_kv_heads, num_q_heads, head_dim, block_size,
+      num_blocks, scale, dtype, out, out_token_stride, nullptr, 0, stream);
+}
+
+extern "C" int nkv_paged_attention_prefill_split(
+    const void* q, int64_t q_token_stride, const void* key_cache, const void* value_cache,
+    const int32_t* block_tables, int64_t table_stride, const int32_t* cu_seqlens_q,
+    const int32_t* cu_seqlens_k, const void* plan, int64_t capacity, int64_t num_seqs,
+    int64_t num_kv_heads, int64_t num_q_heads, int64_t head_dim, int64_t block_size,
+    int64_t num_blocks, float scale, int32_t dtype, void* out, int64_t out_token_stride,
+    void* workspace, int64_t workspace_bytes, void* stream) {
   using namespace nkv;
   if (dtype != NKV_DTYPE_BFLOAT16 && dtype != NKV_DTYPE_FLOAT16) {
     return nkv_fail(NKV_E_INVALID,
@@ -668,19 +952,31 @@ extern "C" int nkv_paged_attention_prefill(
   const int64_t row_bytes = num_kv_heads * head_dim * 2;
   const bool wide = num_blocks * block_size * row_bytes > static_cast<int64_t>(UINT32_MAX);
   const int64_t group = num_q_heads / num_kv_heads;
-  const PrefillKernel kernel =
-      half ? (wide ? prefill_kernel_for<true, true>(group)
-                   : prefill_kernel_for<false, true>(group))
-           : (wide ? prefill_kernel_for<true, false>(group)
-                   : prefill_kernel_for<false, false>(group));
+  const int64_t need = nkv_prefill_workspace_bytes(
+      capacity, num_kv_heads, std::min<int64_t>(table_stride, INT32_MAX) * std::min<int64_t>(block_size, INT32_MAX));
+  const bool split = workspace && need > 0;
+  if (split && (workspace_bytes < need || reinterpret_cast<uint64_t>(workspace) % 16 != 0)) {
+    return nkv_fail(NKV_E_CAPACITY,
+                    "nkv_paged_attention_prefill: workspace of %lld bytes, %lld 16-byte aligned "
+                    "ones needed", static_cast<long long>(workspace_bytes),
+                    static_cast<long long>(need));
+  }
+  const PrefillKernel kernel = wide ? prefill_kernel_for<true>(group, half, split)
+                                    : prefill_kernel_for<false>(group, half, split);
+  const int64_t partials = split_partials(num_kv_heads) * num_kv_heads;
+  float* const part_acc = split ? static_cast<float*>(workspace) : nullptr;
+  f32x2* const part_ml = split ? reinterpret_cast<f32x2*>(part_acc + partials * kPartSums) : nullptr;
+  int2* const tile_parts = split ? reinterpret_cast<int2*>(part_ml + partials * kPfRows) : nullptr;
+  // Workgroups per kv head: one per plan entry, or per piece.
+  const int64_t per_kv_head = split ? split_pieces(num_kv_heads) : capacity;
   int32_t xcd_layout = 0;
-  int64_t grid = capacity * num_kv_heads;
+  int64_t grid = per_kv_head * num_kv_heads;
   if (num_kv_heads % kXcds == 0) {
     xcd_layout = 1;
   } else if (kXcds % num_kv_heads == 0) {
     xcd_layout = 2;
     const int64_t per_head = kXcds / num_kv_heads;
-    grid = kXcds * ((capacity + per_head - 1) / per_head);
+    grid = kXcds * ((per_kv_head + per_head - 1) / per_head);
   }
   if (grid > static_cast<int64_t>(UINT32_MAX / kPfThreads)) {
     return nkv_fail(NKV_E_INVALID, "nkv_paged_attention_prefill: %lld query tiles x %lld kv heads "
@@ -694,6 +990,17 @@ extern "C" int nkv_paged_attention_prefill(
       static_cast<int32_t>(block_size), block_shift, static_cast<int32_t>(num_blocks),
       static_cast<int32_t>(num_kv_heads), cu_seqlens_q, cu_seqlens_k,
       static_cast<const int4*>(plan), static_cast<int32_t>(capacity), xcd_layout,
-      static_cast<int32_t>(num_seqs), scale_log2, static_cast<uint16_t*>(out), out_token_stride);
-  return nkv_check_launch("nkv_paged_attention_prefill");
+      static_cast<int32_t>(num_seqs), scale_log2, static_cast<uint16_t*>(out), out_token_stride,
+      split ? static_cast<int32_t>(per_kv_head) : 0, part_acc, part_ml, tile_parts);
+  if (int rc = nkv_check_launch("nkv_paged_attention_prefill")) return rc;
+  if (!split) return NKV_OK;
+  const auto merge = half ? prefill_merge_kernel<true> : prefill_merge_kernel<false>;
+  const int64_t merge_grid = capacity * num_kv_heads * (kMergeUnits / kMergeWaves);
+  merge<<<dim3(static_cast<unsigned>(merge_grid)), dim3(kMergeWaves * kWave), 0,
+          static_cast<hipStream_t>(stream)>>>(
+      part_acc, part_ml, tile_parts, static_cast<const int4*>(plan),
+      static_cast<int32_t>(num_seqs), cu_seqlens_q, cu_seqlens_k,
+      static_cast<int32_t>(num_kv_heads), static_cast<int32_t>(group),
+      static_cast<uint16_t*>(out), out_token_stride);
+  return nkv_check_launch("nkv_paged_attention_prefill (merge)");
 }

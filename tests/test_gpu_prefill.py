@@ -108,6 +108,49 @@ def test_prefill_matches_oracle(backend, gpu_device, hkv, g, bs):
     check_close(out, *reference(host, scale), f"hkv={hkv} g={g} bs={bs}")
 
 
+@pytest.mark.parametrize("hkv,g,bs,q_lens,k_lens,dtype", [
+    # few query tiles over long contexts: pieces of every length, a last
+    # piece that some rows do not see, tiles of one piece beside cut ones
+    (8, 2, 256, [98, 1, 65, 3], [6001, 700, 2113, 3], torch.bfloat16),
+    (8, 4, 16, [33, 0, 64], [4097, 90, 64], torch.float16),
+    (2, 8, 64, [1, 17, 300], [1, 5000, 300], torch.bfloat16),  # kv heads a divisor of 8
+    (3, 2, 24, [130, 70], [2000, 1290], torch.bfloat16),  # no XCD grouping, 24-row blocks
+    (1, 8, 256, [5], [9000], torch.bfloat16),  # one tile in more pieces than the merge's batch
+    (8, 1, 256, [64] * 4, [513, 512, 511, 577], torch.bfloat16),  # just past the shortest context cut
+    (8, 2, 32, [56 * 64 + 1, 64], [56 * 64 + 1, 1000], torch.bfloat16),  # nearly every slot has a tile
+])
+def test_short_launches_cut_their_keys(backend, gpu_device, hkv, g, bs, q_lens, k_lens, dtype):
+    """Launches of one round of workgroups cut the keys of their query tiles
+    into pieces merged from fp32 partials.  With block ids outside the
+    cache, whose keys drop out, the result is that of the same call without
+    a workspace, which cuts nothing."""
+    from nanokv import _lib
+    from nanokv.paged_kv import ops
+
+    dev, host = build_case(gpu_device, hkv, g, bs, q_lens, k_lens, seed=len(q_lens) + hkv + g, dtype=dtype)
+    scale = 1.0 / math.sqrt(128)
+    out = torch.full_like(dev["q"].contiguous(), float("nan"))
+    run(backend, dev, scale, out=out)
+    ref, ref_abs = reference(host, scale)
+    check_close(out, ref, ref_abs, f"hkv={hkv} g={g} bs={bs} {dtype}")
+
+    for i, n in enumerate(k_lens):
+        if n > 4 * bs:
+            dev["tables"][i, n // bs // 2] = host["kc"].shape[0] + 3
+    run(backend, dev, scale, out=out)
+    plan = backend.build_prefill_plan(dev["q"], dev["kc"], dev["cu_q"], dev["cu_k"])
+    whole = torch.full_like(out, float("nan"))
+    q, kc = dev["q"], dev["kc"]
+    library = _lib.load_library()
+    _lib.check(library.nkv_paged_attention_prefill(
+        q.data_ptr(), q.stride(0), kc.data_ptr(), dev["vc"].data_ptr(), dev["tables"].data_ptr(),
+        dev["tables"].shape[1], dev["cu_q"].data_ptr(), dev["cu_k"].data_ptr(), plan.data_ptr(),
+        plan.shape[0], len(q_lens), hkv, hkv * g, 128, bs, kc.shape[0], scale,
+        ops.DTYPE_CODES[dtype], whole.data_ptr(), whole.stride(0),
+        ops.current_stream_handle(gpu_device)), "prefill without a workspace")
+    check_close(out, whole.float().cpu().numpy(), ref_abs, "dropped blocks")
+
+
 def check_plan(plan, q_lens, k_lens, tile, longest_first):
     """Every query tile exactly once, entries past the tiles empty, and the
     order: most visible keys first (ties in sequence order, each sequence's
