@@ -460,6 +460,25 @@ int nkv_paged_attention_prefill_split(
     int64_t num_blocks, float scale, int32_t dtype, void* out,
     int64_t out_token_stride, void* workspace, int64_t workspace_bytes,
     void* stream);
+/*
+ * The same attention over keys and values that lie back to back, request
+ * after request, with token strides k_token_stride / v_token_stride elements
+ * (multiples of 8, so that views of one fused projection are read in place;
+ * bases 16-byte aligned): flash_attn_varlen_func without a block table, as
+ * Attention.forward calls it for prompts with nothing cached
+ * (nanovllm/layers/attention.py:95-116).  Key t of request i is row
+ * cu_seqlens_k[i] + t of k; rows from max_seqlen_k or total_k_tokens on are
+ * dropped.  Workspace as for max_keys = max_seqlen_k, or null.
+ */
+int nkv_varlen_attention_prefill(
+    const void* q, int64_t q_token_stride, const void* k,
+    int64_t k_token_stride, const void* v, int64_t v_token_stride,
+    int64_t total_k_tokens, int64_t max_seqlen_k, const int32_t* cu_seqlens_q,
+    const int32_t* cu_seqlens_k, const void* plan, int64_t capacity,
+    int64_t num_seqs, int64_t num_kv_heads, int64_t num_q_heads,
+    int64_t head_dim, float scale, int32_t dtype, void* out,
+    int64_t out_token_stride, void* workspace, int64_t workspace_bytes,
+    void* stream);
 
 /*
  * Host-to-device transfer lane: a non-blocking transfer stream (default

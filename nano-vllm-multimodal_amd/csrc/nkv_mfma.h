@@ -86,7 +86,8 @@ __device__ __forceinline__ float row4_sum(float x) {
 // wavefronts read the buffer) before it reads the buffer they fill.
 // M0 is a reserved register, so clang warns that a clobber of it may not be
 // preserved; in the kernels built from this file every M0 access is the
-// s_mov_b32 of these copies (no compiler value lives in M0 across them).
+// s_mov_b32 or s_add_u32 of these copies (no compiler value lives in M0
+// across them).
 // LDS byte address of a __shared__ array (a constant once inlined).
 __device__ __forceinline__ uint32_t lds_address(const u32x4* array) {
   typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
@@ -122,6 +123,24 @@ __device__ __forceinline__ void lds_copy16(const uint8_t* base, uint32_t offset,
                  : "v"(offset), "s"(base), "s"(lds_dst)
                  : "m0", "memory");
   }
+}
+// The same to lds_dst + kDst, the constant added on the way into M0, so that
+// several copies around one LDS address hold one scalar register (a sum
+// computed outside the asm is kept live across a loop: 16 of them pushed the
+// prefill kernel's scalars into lane spills).
+template <int kDst>
+__device__ __forceinline__ void lds_copy16_at(const uint8_t* src, uint32_t lds_dst) {
+  asm volatile("s_add_u32 m0, %1, %2\n\tglobal_load_lds_dwordx4 %0, off"
+               :
+               : "v"(src), "s"(lds_dst), "n"(kDst)
+               : "m0", "scc", "memory");
+}
+template <int kDst>
+__device__ __forceinline__ void lds_copy16_at(const uint8_t* base, uint32_t offset, uint32_t lds_dst) {
+  asm volatile("s_add_u32 m0, %2, %3\n\tglobal_load_lds_dwordx4 %0, %1"
+               :
+               : "v"(offset), "s"(base), "s"(lds_dst), "n"(kDst)
+               : "m0", "scc", "memory");
 }
 
 // Four consecutive elements of V^T for the PV product: lane 16 G + 4 j + q

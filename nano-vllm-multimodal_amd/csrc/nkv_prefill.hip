@@ -74,7 +74,12 @@ constexpr int kTileChunks = kPfKeys * 16;  // 16-byte chunks per K or V tile
 // longest workgroups start first and the short ones fill the tail; ties in
 // plan order.  Plans of up to kPfSortMax tiles are sorted in LDS by one
 // workgroup (bitonic); longer ones list each sequence's tiles last tile
-// first, sequence after sequence.
+// first, sequence after sequence.  With up to kPfRankSeqs sequences, as a
+// prefill step has, nothing is sorted: a sequence's tiles are evenly spaced
+// in what they see, so the tiles of sequence j ahead of a given tile are
+// counted from its lengths, and the count over all sequences is the tile's
+// place (no barriers: 457 tiles took 12 us sorted, 45 passes of the
+// network; a tile's place costs some 20 instructions per sequence).
 #ifndef NKV_PF_SETPRIO
 #define NKV_PF_SETPRIO 1  // raise the wave's priority over its MFMA block (0: never)
 #endif
@@ -82,6 +87,7 @@ constexpr int kTileChunks = kPfKeys * 16;  // 16-byte chunks per K or V tile
 #define NKV_PF_SORT_MAX 2048  // longest plan sorted in LDS (0: never sort)
 #endif
 constexpr int kPfSortMax = NKV_PF_SORT_MAX;
+constexpr int kPfRankSeqs = 128;
 
 __global__ __launch_bounds__(kPfPlanThreads) void prefill_plan_kernel(
     const int32_t* __restrict__ cu_seqlens_q, const int32_t* __restrict__ cu_seqlens_k,
@@ -108,6 +114,39 @@ __global__ __launch_bounds__(kPfPlanThreads) void prefill_plan_kernel(
     const int32_t visible = max(0, cu_seqlens_k[i + 1] - cu_seqlens_k[i] - len + t0 + ntok);
     return make_int4(i, t0, ntok, visible / kPfKeys + (visible % kPfKeys != 0 ? 1 : 0));
   };
+  if (sort && total <= kPfSortMax && num_seqs <= kPfRankSeqs) {  // one workgroup
+    int32_t* s_len = s_tmp + kPfPlanThreads / 64 + 1;  // [num_seqs] queries
+    int32_t* s_cached = s_len + num_seqs;              // [num_seqs] keys before the first query
+    for (int32_t j = threadIdx.x; j < num_seqs; j += kPfPlanThreads) {
+      s_len[j] = cu_seqlens_q[j + 1] - cu_seqlens_q[j];
+      s_cached[j] = cu_seqlens_k[j + 1] - cu_seqlens_k[j] - s_len[j];
+    }
+    __syncthreads();
+    for (int32_t e = threadIdx.x; e < capacity || e < total; e += kPfPlanThreads) {
+      if (e >= total) {
+        plan[e] = make_int4(0, 0, 0, 0);
+        continue;
+      }
+      const int4 en = entry_of(e);
+      const int32_t visible = max(0, s_cached[en.x] + en.y + en.z);
+      int32_t place = e - s_first[en.x];  // this sequence's later tiles
+      for (int32_t j = 0; j < num_seqs; ++j) {
+        if (j == en.x) continue;
+        // Tiles of sequence j that see at least `floor` keys; tile t sees
+        // cached + min(len, (t + 1) tile_tokens), but never less than 0.
+        const int64_t floor = static_cast<int64_t>(visible) + (j > en.x ? 1 : 0);
+        const int32_t tiles = s_first[j + 1] - s_first[j];
+        const int64_t own = floor - s_cached[j];  // of its own queries
+        if (floor <= 0 || own <= tile_tokens) {
+          place += floor <= 0 || own <= s_len[j] ? tiles : 0;
+        } else if (own <= s_len[j]) {
+          place += tiles - (static_cast<int32_t>(own) - 1) / tile_tokens;
+        }
+      }
+      if (place < capacity) plan[place] = en;
+    }
+    return;
+  }
   if (sort && total <= kPfSortMax) {  // one workgroup (the launch makes sure)
     // Sort keys: (2^31 - 1 - visible keys) << 32 | e, ascending; padding last.
     const int32_t key_offset = (num_seqs + kPfPlanThreads / 64 + 3) & ~1;  // 8-byte aligned
@@ -155,10 +194,17 @@ __global__ __launch_bounds__(kPfPlanThreads) void prefill_plan_kernel(
 }
 
 // Where one sequence's context rows live: its block table and the cache
-// geometry.  Power-of-two block sizes map rows with shifts.
+// geometry.  Power-of-two block sizes map rows with shifts.  Keys without a
+// table use the same arithmetic: the "table" is the sequence's entry of
+// cu_seqlens_k, its first row, looked up at index 0 for every key, and the
+// key is the offset (index_mask 0, offset_mask all ones): a
+// branch between the two would wait for the early table load, and with it
+// for every copy in flight, where its sides join.
 struct ContextMap {
   const int32_t* table;
   int64_t table_stride;
+  int32_t index_mask;   // all ones, or 0
+  int32_t offset_mask;  // block_size - 1 when that is a mask, or all ones
   int32_t block_size;
   int32_t block_shift;  // log2(block_size), or -1 when it is not a power of two
   int32_t num_blocks;
@@ -170,14 +216,14 @@ struct ContextMap {
   __device__ __forceinline__ int32_t block_of(int32_t t) const {
     const int32_t logical = block_shift >= 0 ? t >> block_shift : t / block_size;
     if (t >= num_keys || logical >= table_stride) return -1;
-    return table[logical];
+    return table[logical & index_mask];
   }
   __device__ __forceinline__ int32_t row_in(int32_t t, int32_t block) const {
     if (block < 0 || block >= num_blocks) return -1;
-    const int32_t offset = block_shift >= 0 ? t & (block_size - 1) : t % block_size;
-    return block * block_size + offset;  // num_blocks * block_size <= INT32_MAX
+    const int32_t offset = block_shift >= 0 ? t & offset_mask : t % block_size;
+    const int32_t row = block * block_size + offset;  // num_blocks * block_size <= INT32_MAX
+    return row < num_blocks * block_size ? row : -1;  // (keys without a table may run past the end)
   }
-  __device__ __forceinline__ int32_t row(int32_t t) const { return row_in(t, block_of(t)); }
 };
 
 // Wavefront 0 resolves the 64 rows of the tile starting at key0 (one per
@@ -206,19 +252,32 @@ __device__ __forceinline__ void issue_copies(const u32x4* dst, const int32_t* ro
   int32_t row[kCopies];
 #pragma unroll
   for (int i = 0; i < kCopies; ++i) row[i] = rows[kKeysPerWave * wave + 4 * i + (lane >> 4)];
-#pragma unroll
-  for (int i = 0; i < kCopies; ++i) {
-    const int key0 = kKeysPerWave * wave + 4 * i;
-    const int key = key0 + (lane >> 4);
+  const uint32_t lds_dst = lds_address(dst) + kKeysPerWave * 256 * wave;  // wave is uniform
+  auto copy = [&](auto index) {
+    constexpr int i = decltype(index)::value;
+    const int key = kKeysPerWave * wave + 4 * i + (lane >> 4);
     const uint32_t chunk = 16u * (kValue ? pos ^ ((key & 7) << 1) : pos ^ (key & 15));
-    const uint32_t lds_dst = lds_address(dst) + key0 * 256;  // wave is uniform
     if (row[i] >= 0) {
       if (kWide) {
-        lds_copy16(head_base + static_cast<int64_t>(row[i]) * row_bytes + chunk, lds_dst);
+        lds_copy16_at<1024 * i>(
+            head_base + (static_cast<uint64_t>(static_cast<uint32_t>(row[i])) * row_bytes + chunk), lds_dst);
       } else {
-        lds_copy16(head_base, static_cast<uint32_t>(row[i]) * row_bytes + chunk, lds_dst);
+        // The empty asm keeps product and sum apart: as one 64-bit
+        // multiply-add its unused upper addend may be any register, and one
+        // with a load in flight (the block id fetched ahead) makes the copy
+        // wait for every copy before it (85 us became 94).
+        uint32_t at = static_cast<uint32_t>(row[i]) * row_bytes;
+        asm("" : "+v"(at));
+        lds_copy16_at<1024 * i>(head_base, at + chunk, lds_dst);
       }
     }
+  };
+  static_assert(kCopies == 4 || kCopies == 2, "4 or 8 waves");
+  copy(std::integral_constant<int, 0>{});
+  copy(std::integral_constant<int, 1>{});
+  if constexpr (kCopies == 4) {
+    copy(std::integral_constant<int, 2>{});
+    copy(std::integral_constant<int, 3>{});
   }
 }
 
@@ -473,6 +532,7 @@ template <int G, bool kWide, bool kHalf, bool kSplit>
 __global__ __launch_bounds__(kPfThreads, kPfBlocksPerCU) void attn_prefill_kernel(
     const uint16_t* __restrict__ q, int64_t q_token_stride,
     const uint8_t* __restrict__ key_cache, const uint8_t* __restrict__ value_cache,
+    uint32_t k_row_bytes, uint32_t v_row_bytes,
     const int32_t* __restrict__ tables, int64_t table_stride, int32_t block_size,
     int32_t block_shift, int32_t num_blocks, int32_t num_kv_heads,
     const int32_t* __restrict__ cu_seqlens_q, const int32_t* __restrict__ cu_seqlens_k,
@@ -520,14 +580,15 @@ __global__ __launch_bounds__(kPfThreads, kPfBlocksPerCU) void attn_prefill_kerne
   const int lane = tid % kWave;
   const int c16 = lane & 15;  // the lane's query row inside a 16-row block
   const int g4 = lane >> 4;   // which quarter of the MFMA k dimension the lane holds
-  const uint32_t row_bytes = static_cast<uint32_t>(num_kv_heads) * kPfDim * 2;
   const uint8_t* const k_head = key_cache + static_cast<int64_t>(kh) * kPfDim * 2;
   const uint8_t* const v_head = value_cache + static_cast<int64_t>(kh) * kPfDim * 2;
   // keys the last row sees (<= lk); every row sees at least first_row_keys
   const int32_t num_keys = lk - lq + tok0 + ntok;
   const int32_t first_row_keys = lk - lq + tok0 + 1;
-  const ContextMap map{tables + static_cast<int64_t>(seq) * table_stride, table_stride,
-                       block_size, block_shift, num_blocks, num_keys};
+  const bool paged = tables != nullptr;
+  const ContextMap map{paged ? tables + static_cast<int64_t>(seq) * table_stride : cu_seqlens_k + seq,
+                       table_stride, paged ? -1 : 0, paged ? block_size - 1 : -1, block_size,
+                       block_shift, num_blocks, num_keys};
 
   // Q^T operands (B of S^T = K Q^T): lane holds row m, dims 32 * dc + 8 * g4 .. +8.
   X8 qb[2][4];
@@ -598,9 +659,9 @@ __global__ __launch_bounds__(kPfThreads, kPfBlocksPerCU) void attn_prefill_kerne
     }
   }
   __syncthreads();
-  issue_copies<kWide, false>(k_buf0, rows_buf[0], k_head, row_bytes, wave, lane);
-  issue_copies<kWide, true>(v_buf0, rows_buf[0], v_head, row_bytes, wave, lane);
-  if (num_tiles > 1) issue_copies<kWide, false>(k_buf1, rows_buf[1], k_head, row_bytes, wave, lane);
+  issue_copies<kWide, false>(k_buf0, rows_buf[0], k_head, k_row_bytes, wave, lane);
+  issue_copies<kWide, true>(v_buf0, rows_buf[0], v_head, v_row_bytes, wave, lane);
+  if (num_tiles > 1) issue_copies<kWide, false>(k_buf1, rows_buf[1], k_head, k_row_bytes, wave, lane);
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
   const int tr_key = 4 * g4 + ((lane >> 2) & 3);  // key this lane addresses in a V^T read (of 16)
@@ -650,10 +711,10 @@ __global__ __launch_bounds__(kPfThreads, kPfBlocksPerCU) void attn_prefill_kerne
       if (tile + 4 < num_tiles) ahead_block = map.block_of(key0 + 4 * kPfKeys + lane);
     }
     if (tile + 2 < num_tiles) {
-      issue_copies<kWide, false>(k_this, rows_buf[(tile + 2) & 3], k_head, row_bytes, wave, lane);
+      issue_copies<kWide, false>(k_this, rows_buf[(tile + 2) & 3], k_head, k_row_bytes, wave, lane);
     }
     if (tile + 1 < num_tiles) {
-      issue_copies<kWide, true>(v_next, rows_buf[(tile + 1) & 3], v_head, row_bytes, wave, lane);
+      issue_copies<kWide, true>(v_next, rows_buf[(tile + 1) & 3], v_head, v_row_bytes, wave, lane);
     }
     // A tile is plain when every row sees all its keys and all are valid:
     // its scores need no mask.
@@ -671,7 +732,13 @@ __global__ __launch_bounds__(kPfThreads, kPfBlocksPerCU) void attn_prefill_kerne
           const int32_t row[4] = {r.x, r.y, r.z, r.w};
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            if (key0 + 16 * kb + 4 * g4 + i > limit[mb] || row[i] < 0) st[kb][mb][i] = -INFINITY;
+            // Negative when the key is past the limit or its row is -1.
+            // Selected by its sign bits: 32 comparisons would hold 32 scalar
+            // register pairs and push the loop's scalars into lane spills.
+            const uint32_t hidden =
+                static_cast<uint32_t>(((limit[mb] - (key0 + 16 * kb + 4 * g4 + i)) | row[i]) >> 31);
+            st[kb][mb][i] = __uint_as_float((hidden & 0xFF800000u) |  // -inf
+                                            (~hidden & __float_as_uint(st[kb][mb][i])));
           }
         }
       }
@@ -789,8 +856,8 @@ __global__ __launch_bounds__(kPfThreads, kPfBlocksPerCU) void attn_prefill_kerne
   }
 }
 
-using PrefillKernel = void (*)(const uint16_t*, int64_t, const uint8_t*, const uint8_t*,
-                               const int32_t*, int64_t, int32_t, int32_t, int32_t, int32_t,
+using PrefillKernel = void (*)(const uint16_t*, int64_t, const uint8_t*, const uint8_t*, uint32_t,
+                               uint32_t, const int32_t*, int64_t, int32_t, int32_t, int32_t, int32_t,
                                const int32_t*, const int32_t*, const int4*, int32_t, int32_t,
                                int32_t, float, uint16_t*, int64_t, int32_t, float*, f32x2*, int2*);
 
@@ -856,7 +923,9 @@ extern "C" int nkv_build_prefill_plan(const int32_t* cu_seqlens_q, const int32_t
   const bool sort = capacity <= kPfSortMax;
   const int64_t blocks = sort ? 1 : (capacity + kPfPlanThreads - 1) / kPfPlanThreads;
   const size_t scan_ints = static_cast<size_t>(num_seqs) + 1 + kPfPlanThreads / kWave + 1;
-  const size_t lds = sort ? ((scan_ints + 1) & ~size_t{1}) * sizeof(int32_t) +
+  const size_t lds = sort && num_seqs <= kPfRankSeqs
+                         ? (scan_ints + 2 * static_cast<size_t>(num_seqs)) * sizeof(int32_t)
+                     : sort ? ((scan_ints + 1) & ~size_t{1}) * sizeof(int32_t) +
                                 kPfSortMax * sizeof(uint64_t)
                           : scan_ints * sizeof(int32_t);
   prefill_plan_kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(kPfPlanThreads), lds,
@@ -877,27 +946,19 @@ extern "C" int64_t nkv_prefill_workspace_bytes(int64_t capacity, int64_t num_kv_
   return partials * (kPartSums * 4 + kPfRows * 8) + capacity * 8;
 }
 
-extern "C" int nkv_paged_attention_prefill(
-    const void* q, int64_t q_token_stride, const void* key_cache, const void* value_cache,
-    const int32_t* block_tables, int64_t table_stride, const int32_t* cu_seqlens_q,
-    const int32_t* cu_seqlens_k, const void* plan, int64_t capacity, int64_t num_seqs,
-    int64_t num_kv_heads, int64_t num_q_heads, int64_t head_dim, int64_t block_size,
-    int64_t num_blocks, float scale, int32_t dtype, void* out, int64_t out_token_stride,
-    void* stream) {
-  return nkv_paged_attention_prefill_split(
-      q, q_token_stride, key_cache, value_cache, block_tables, table_stride, cu_seqlens_q,
-      cu_seqlens_k, plan, capacity, num_seqs, num_kv_heads, num_q_heads, head_dim, block_size,
-      num_blocks, scale, dtype, out, out_token_stride, nullptr, 0, stream);
-}
+namespace nkv {
+namespace {
 
-extern "C" int nkv_paged_attention_prefill_split(
-    const void* q, int64_t q_token_stride, const void* key_cache, const void* value_cache,
-    const int32_t* block_tables, int64_t table_stride, const int32_t* cu_seqlens_q,
-    const int32_t* cu_seqlens_k, const void* plan, int64_t capacity, int64_t num_seqs,
-    int64_t num_kv_heads, int64_t num_q_heads, int64_t head_dim, int64_t block_size,
-    int64_t num_blocks, float scale, int32_t dtype, void* out, int64_t out_token_stride,
-    void* workspace, int64_t workspace_bytes, void* stream) {
-  using namespace nkv;
+// Both prefill entries.  Keys are rows of the paged caches (block_tables),
+// or, without tables, rows of k and v themselves (block_size 1, num_blocks
+// rows, table_stride the longest context).  Strides in elements.
+int run_prefill(const void* q, int64_t q_token_stride, const void* key_cache, int64_t k_row_stride,
+                const void* value_cache, int64_t v_row_stride, const int32_t* block_tables,
+                bool has_tables, int64_t table_stride, const int32_t* cu_seqlens_q,
+                const int32_t* cu_seqlens_k, const void* plan, int64_t capacity, int64_t num_seqs,
+                int64_t num_kv_heads, int64_t num_q_heads, int64_t head_dim, int64_t block_size,
+                int64_t num_blocks, float scale, int32_t dtype, void* out, int64_t out_token_stride,
+                void* workspace, int64_t workspace_bytes, void* stream) {
   if (dtype != NKV_DTYPE_BFLOAT16 && dtype != NKV_DTYPE_FLOAT16) {
     return nkv_fail(NKV_E_INVALID,
                     "nkv_paged_attention_prefill: only bfloat16 and float16 are supported");
@@ -927,7 +988,7 @@ extern "C" int nkv_paged_attention_prefill_split(
   }
   if (num_seqs == 0 || capacity == 0) return NKV_OK;
   if (!q || !key_cache || !value_cache || !out || !plan || !cu_seqlens_q || !cu_seqlens_k ||
-      (table_stride > 0 && !block_tables)) {
+      (has_tables && table_stride > 0 && !block_tables)) {
     return nkv_fail(NKV_E_INVALID, "nkv_paged_attention_prefill: null pointer");
   }
   if ((reinterpret_cast<uint64_t>(q) | reinterpret_cast<uint64_t>(key_cache) |
@@ -949,7 +1010,7 @@ extern "C" int nkv_paged_attention_prefill_split(
   }
   // Byte offsets of rows into one cache fit 32 bits unless the cache is
   // larger than 4 GiB; then the copies form 64-bit addresses.
-  const int64_t row_bytes = num_kv_heads * head_dim * 2;
+  const int64_t row_bytes = 2 * std::max(k_row_stride, v_row_stride);
   const bool wide = num_blocks * block_size * row_bytes > static_cast<int64_t>(UINT32_MAX);
   const int64_t group = num_q_heads / num_kv_heads;
   const int64_t need = nkv_prefill_workspace_bytes(
@@ -986,7 +1047,8 @@ extern "C" int nkv_paged_attention_prefill_split(
   kernel<<<dim3(static_cast<unsigned>(grid)), dim3(kPfThreads), 0,
            static_cast<hipStream_t>(stream)>>>(
       static_cast<const uint16_t*>(q), q_token_stride, static_cast<const uint8_t*>(key_cache),
-      static_cast<const uint8_t*>(value_cache), block_tables, table_stride,
+      static_cast<const uint8_t*>(value_cache), static_cast<uint32_t>(2 * k_row_stride),
+      static_cast<uint32_t>(2 * v_row_stride), has_tables ? block_tables : nullptr, table_stride,
       static_cast<int32_t>(block_size), block_shift, static_cast<int32_t>(num_blocks),
       static_cast<int32_t>(num_kv_heads), cu_seqlens_q, cu_seqlens_k,
       static_cast<const int4*>(plan), static_cast<int32_t>(capacity), xcd_layout,
@@ -1003,4 +1065,55 @@ extern "C" int nkv_paged_attention_prefill_split(
       static_cast<int32_t>(num_kv_heads), static_cast<int32_t>(group),
       static_cast<uint16_t*>(out), out_token_stride);
   return nkv_check_launch("nkv_paged_attention_prefill (merge)");
+}
+
+}  // namespace
+}  // namespace nkv
+
+extern "C" int nkv_paged_attention_prefill(
+    const void* q, int64_t q_token_stride, const void* key_cache, const void* value_cache,
+    const int32_t* block_tables, int64_t table_stride, const int32_t* cu_seqlens_q,
+    const int32_t* cu_seqlens_k, const void* plan, int64_t capacity, int64_t num_seqs,
+    int64_t num_kv_heads, int64_t num_q_heads, int64_t head_dim, int64_t block_size,
+    int64_t num_blocks, float scale, int32_t dtype, void* out, int64_t out_token_stride,
+    void* stream) {
+  return nkv_paged_attention_prefill_split(
+      q, q_token_stride, key_cache, value_cache, block_tables, table_stride, cu_seqlens_q,
+      cu_seqlens_k, plan, capacity, num_seqs, num_kv_heads, num_q_heads, head_dim, block_size,
+      num_blocks, scale, dtype, out, out_token_stride, nullptr, 0, stream);
+}
+
+extern "C" int nkv_paged_attention_prefill_split(
+    const void* q, int64_t q_token_stride, const void* key_cache, const void* value_cache,
+    const int32_t* block_tables, int64_t table_stride, const int32_t* cu_seqlens_q,
+    const int32_t* cu_seqlens_k, const void* plan, int64_t capacity, int64_t num_seqs,
+    int64_t num_kv_heads, int64_t num_q_heads, int64_t head_dim, int64_t block_size,
+    int64_t num_blocks, float scale, int32_t dtype, void* out, int64_t out_token_stride,
+    void* workspace, int64_t workspace_bytes, void* stream) {
+  const int64_t row = num_kv_heads * head_dim;
+  return nkv::run_prefill(q, q_token_stride, key_cache, row, value_cache, row, block_tables, true,
+                          table_stride, cu_seqlens_q, cu_seqlens_k, plan, capacity, num_seqs,
+                          num_kv_heads, num_q_heads, head_dim, block_size, num_blocks, scale, dtype,
+                          out, out_token_stride, workspace, workspace_bytes, stream);
+}
+
+extern "C" int nkv_varlen_attention_prefill(
+    const void* q, int64_t q_token_stride, const void* k, int64_t k_token_stride, const void* v,
+    int64_t v_token_stride, int64_t total_k_tokens, int64_t max_seqlen_k,
+    const int32_t* cu_seqlens_q, const int32_t* cu_seqlens_k, const void* plan, int64_t capacity,
+    int64_t num_seqs, int64_t num_kv_heads, int64_t num_q_heads, int64_t head_dim, float scale,
+    int32_t dtype, void* out, int64_t out_token_stride, void* workspace, int64_t workspace_bytes,
+    void* stream) {
+  using namespace nkv;
+  const int64_t row = num_kv_heads * head_dim;
+  if (k_token_stride < row || v_token_stride < row || k_token_stride > INT32_MAX ||
+      v_token_stride > INT32_MAX || (k_token_stride | v_token_stride) % 8 != 0) {
+    return nkv_fail(NKV_E_INVALID,
+                    "nkv_varlen_attention_prefill: k and v token strides must hold a row and be "
+                    "multiples of 8 elements");
+  }
+  return run_prefill(q, q_token_stride, k, k_token_stride, v, v_token_stride, nullptr, false,
+                     max_seqlen_k, cu_seqlens_q, cu_seqlens_k, plan, capacity, num_seqs,
+                     num_kv_heads, num_q_heads, head_dim, 1, total_k_tokens, scale, dtype, out,
+                     out_token_stride, workspace, workspace_bytes, stream);
 }

@@ -21,6 +21,7 @@ import torch
 
 from nanokv.paged_kv.base import index_value_validation_enabled
 from nanokv.paged_kv.hip_backend import HIPPagedKVBackend
+from nanokv.paged_kv.ops import varlen_attention_prefill, varlen_prefill_in_place
 
 _BACKEND = HIPPagedKVBackend()
 _UNSUPPORTED_DEFAULTS = {
@@ -55,11 +56,21 @@ def flash_attn_varlen_func(q, k, v, max_seqlen_q, cu_seqlens_q, max_seqlen_k, cu
     _check_options("flash_attn_varlen_func", causal, options)
     scale = 1.0 / math.sqrt(q.shape[-1]) if softmax_scale is None else float(softmax_scale)
     if block_table is None:
-        # Contiguous keys: a cache of one-row blocks whose table for request
-        # i counts up from cu_seqlens_k[i] (entries past its length are
-        # never read).
         if k.ndim != 3 or v.shape != k.shape:
             raise ValueError("without block_table, k and v must be [total_k, kv_heads, head_dim]")
+        # Keys back to back are read where they lie, views of the fused
+        # projection included: compacting them, building a table for them
+        # and sorting the plan were five launches beside the attention,
+        # 23 us of a 1,511-token prompt's 62.  (The host-side value checks
+        # of index validation belong to the paged path.)
+        if (not index_value_validation_enabled(cu_seqlens_k)
+                and varlen_prefill_in_place(q, k, v, cu_seqlens_q, cu_seqlens_k)):
+            _BACKEND._load()
+            return varlen_attention_prefill(q, k, v, cu_seqlens_q, cu_seqlens_k,
+                                            max(1, int(max_seqlen_k)), scale)
+        # Otherwise: a cache of one-row blocks whose table for request i
+        # counts up from cu_seqlens_k[i] (entries past its length are never
+        # read).
         k_cache = k.contiguous().unsqueeze(1)
         v_cache = v.contiguous().unsqueeze(1)
         width = max(1, int(max_seqlen_k))

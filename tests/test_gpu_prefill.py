@@ -421,6 +421,71 @@ def test_flash_varlen_contiguous_keys_matches_oracle(gpu_device):
     check_close(out, *reference(host, 0.1), "flash varlen contiguous")
 
 
+@pytest.mark.parametrize("hkv,g,q_lens,k_lens,layout", [
+    (2, 8, [1511], [1511], "fused"),        # one prompt, keys cut into pieces
+    (8, 2, [70, 5, 129], [70, 5, 129], "fused"),
+    (4, 7, [1, 0, 300, 19], [40, 7, 900, 19], "kv"),  # fewer queries than keys; k and v of one tensor
+    (3, 1, [64, 65], [64, 65], "own"),      # tensors of their own, no XCD grouping
+    (1, 4, [33, 1], [2000, 513], "own"),
+    (2, 3, [50, 60], [50, 60], "odd"),      # rows 8 bytes off 16: the paged path compacts them
+    (2, 2, [40, 30], [90, 30], "short"),    # max_seqlen_k below a length: its last keys drop out
+])
+def test_flash_varlen_in_place_equals_the_paged_path(gpu_device, monkeypatch, hkv, g, q_lens, k_lens, layout):
+    """Keys back to back, read where they lie: against the oracle, and equal
+    to the same call through a table of one-row blocks."""
+    from nanokv import flash
+
+    dev, host = build_case(gpu_device, hkv, g, 16, q_lens, k_lens, seed=hkv * 10 + g)
+    total = sum(k_lens)
+    rows = [np.concatenate([oracle.gather(host[c], host["tables"][i], n) for i, n in enumerate(k_lens)])
+            for c in ("kc", "vc")]
+    k, v = (torch.from_numpy(r).view(torch.bfloat16).to(gpu_device) for r in rows)
+    width = hkv * 128
+    if layout == "fused":
+        buf = torch.zeros((total, (g + 2) * width), dtype=torch.bfloat16, device=gpu_device)
+        views = [buf[:, g * width:(g + 1) * width], buf[:, (g + 1) * width:]]
+    elif layout == "kv":
+        buf = torch.zeros((2, total, width + 8), dtype=torch.bfloat16, device=gpu_device)
+        views = [buf[0, :, :width], buf[1, :, 8:]]
+    elif layout == "odd":
+        buf = torch.zeros((2, total, width + 4), dtype=torch.bfloat16, device=gpu_device)
+        views = [buf[0, :, :width], buf[1, :, 4:]]
+    else:
+        views = [torch.empty_like(k).view(total, width), torch.empty_like(v).view(total, width)]
+    for view, rows_of in zip(views, (k, v)):
+        view.copy_(rows_of.view(total, width))
+    k, v = (view.unflatten(1, (hkv, 128)) for view in views)
+    assert flash.varlen_prefill_in_place(dev["q"], k, v, dev["cu_q"], dev["cu_k"]) == (layout != "odd")
+    max_k = max(k_lens) - (21 if layout == "short" else 0)
+
+    def call():
+        return flash.flash_attn_varlen_func(dev["q"], k, v, max(q_lens), dev["cu_q"], max_k, dev["cu_k"],
+                                            softmax_scale=0.1, causal=True)
+
+    out = call()
+    if layout != "short":
+        check_close(out, *reference(host, 0.1), f"{layout} hkv={hkv} g={g}")
+    monkeypatch.setattr(flash, "varlen_prefill_in_place", lambda *a: False)
+    assert torch.equal(out, call())
+
+
+@pytest.mark.parametrize("num_seqs,mean_tokens,group", [(1, 8192, 7), (128, 60, 8), (129, 60, 8), (16, 5, 1)])
+def test_plan_order_ranked_and_sorted(gpu_device, num_seqs, mean_tokens, group):
+    """Both ways of ordering a plan: places counted from the lengths (up to
+    128 requests) and the sort (more), with many equal tiles."""
+    from nanokv import _lib
+    from nanokv.paged_kv import ops
+
+    rng = np.random.default_rng(num_seqs)
+    q_lens = [mean_tokens] if num_seqs == 1 else rng.integers(0, 2 * mean_tokens, num_seqs).tolist()
+    k_lens = [q + 16 * int(c) for q, c in zip(q_lens, rng.integers(0, 4, num_seqs))]
+    cu = [torch.tensor(np.concatenate([[0], np.cumsum(n)]), dtype=torch.int32, device=gpu_device)
+          for n in (q_lens, k_lens)]
+    plan = ops.build_prefill_plan(*cu, sum(q_lens), group).cpu().numpy()
+    check_plan(plan, q_lens, k_lens, int(_lib.load_library().nkv_prefill_tile_tokens(group)),
+               longest_first=True)
+
+
 def check_decode(out, host, lengths, scale, what):
     """Decode output [batch, 1, heads, 128] against the oracle within
     1e-3 + 2^-8 (ref_abs + |ref|), ref_abs being the same attention over |V|
