@@ -395,6 +395,17 @@ int nkv_paged_attention_decode(const void* q, int64_t q_seq_stride,
                                int64_t num_blocks, float scale, int32_t dtype,
                                void* workspace, int64_t workspace_bytes,
                                void* out, int64_t out_seq_stride, void* stream);
+/* The same with the total context tokens (the plan's; -1: unknown), which
+ * bound the entry split's launch: without them it has a workgroup for every
+ * entry the plan could hold. */
+int nkv_paged_attention_decode_total(
+    const void* q, int64_t q_seq_stride, const void* key_cache,
+    const void* value_cache, const int32_t* block_tables, int64_t table_stride,
+    const void* plan, int64_t capacity, const int32_t* first_part,
+    int64_t num_seqs, int64_t num_kv_heads, int64_t num_q_heads,
+    int64_t head_dim, int64_t block_size, int64_t num_blocks, float scale,
+    int32_t dtype, void* workspace, int64_t workspace_bytes, void* out,
+    int64_t out_seq_stride, int64_t total_tokens, void* stream);
 
 /*
  * Paged-attention prefill: causal attention of each sequence's chunk of

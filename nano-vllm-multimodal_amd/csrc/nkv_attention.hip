@@ -31,6 +31,7 @@
 // The G = Hq / Hkv query heads of one kv head are the 16 columns of MFMA
 // tiles (G <= 16), so a chunk costs the same 13 MFMAs whatever G is (see
 // attn_decode_range_kernel).
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 
@@ -399,6 +400,30 @@ __device__ __forceinline__ void emit_partial(uint32_t* acc_out, f32x2* ml_out, f
   if (lane == 0) store_stream(ml_out, f32x2{mm + static_cast<float>(k), lsum * down});
 }
 
+// Entries of 768 rows leave most of the chip idle when the contexts are
+// short or few: one sequence of 5,003 rows is 7 entries, 56 workgroups of 8
+// kv heads, each walking 12 chunks per wave in a row.  Such a launch cuts
+// every entry in 2 where that makes at most kHalvesTarget workgroups (four
+// rounds of two per CU: 920 workgroups are 1.8 rounds, 1,840 halves pack
+// better, 12 layers of a 30-sequence step 782 -> 752 us), and further, up to
+// 16, where that makes at most kPartsTarget (shorter parts cost more to start
+// than they balance: 23 sequences of 34k rows, 944 halves 31.5 us, 1,888
+// quarters 33.6).  The parts must fit the plan's capacity, which the partials
+// are numbered in: part p of n of entry e writes partial e n + p.  The
+// partial and the reduce kernel take n from the plan's entry total alike.
+constexpr int kHalvesTarget = 2048;
+constexpr int kPartsTarget = 1024;
+constexpr int kMaxSub = 16;
+__device__ __forceinline__ int32_t entry_parts(int32_t entries, int32_t num_kv_heads, int64_t capacity) {
+  const int64_t groups = static_cast<int64_t>(entries) * num_kv_heads;
+  int32_t n = 1;
+  while (n < kMaxSub && groups * 2 * n <= (n == 1 ? kHalvesTarget : kPartsTarget) &&
+         static_cast<int64_t>(entries) * 2 * n <= capacity) {
+    n *= 2;
+  }
+  return n;
+}
+
 // One wavefront's LDS: its ring while it runs, its partials afterwards.
 union EntryWaveMem {
   struct {
@@ -416,9 +441,11 @@ struct EntryShared {
   int32_t rows[(kEntryRows + kDecKeys - 1) / kDecKeys * kDecKeys];  // whole chunks
 };
 
+// Item `item` of the launch: kv head item % Hkv (rotated) of part
+// item / Hkv, itself part % subs of entry part / subs.
 template <bool kWide, bool kHalf>
-__global__ __launch_bounds__(kDecThreads) void attn_decode_entry_kernel(
-    const uint16_t* __restrict__ q, int64_t q_seq_stride,
+__device__ __forceinline__ void decode_entry(
+    EntryShared& sh, int64_t item, int32_t subs, const uint16_t* __restrict__ q, int64_t q_seq_stride,
     const uint8_t* __restrict__ key_cache, const uint8_t* __restrict__ value_cache,
     const int32_t* __restrict__ tables, int64_t table_stride, int32_t block_size,
     int32_t num_blocks, int32_t num_kv_heads, int32_t group, const int4* __restrict__ plan,
@@ -428,7 +455,6 @@ __global__ __launch_bounds__(kDecThreads) void attn_decode_entry_kernel(
   typedef typename E::T T;
   typedef typename E::X8 X8;
   typedef typename E::X4 X4;
-  __shared__ EntryShared sh;
 
   // The kv head rotates with the entry.  Workgroups are dealt to the 8 XCDs
   // round-robin (blockIdx % 8), so head blockIdx % Hkv would pin each XCD to
@@ -438,17 +464,20 @@ __global__ __launch_bounds__(kDecThreads) void attn_decode_entry_kernel(
   // rotated).  Workgroups of one XCD with the same blockIdx % Hkv are
   // `period` entries apart, so adding part / period walks them over every
   // head; for a fixed entry the heads stay a permutation.
-  const int64_t part = blockIdx.x / num_kv_heads;
+  const int64_t part = item / num_kv_heads;
   const int32_t period = 8 / min(8, num_kv_heads & -num_kv_heads);  // 8 / gcd(Hkv, 8)
   const int32_t kh =
-      static_cast<int32_t>((blockIdx.x % num_kv_heads + part / period) % num_kv_heads);
-  const int4 entry = plan[part];
-  const int32_t row0 = entry.x;
+      static_cast<int32_t>((item % num_kv_heads + part / period) % num_kv_heads);
+  const int4 entry = plan[part / subs];
+  // This part's rows of the entry: equal shares of whole chunks.
+  const int32_t share = ((entry.y + subs - 1) / subs + kDecKeys - 1) / kDecKeys * kDecKeys;
+  const int32_t skip = static_cast<int32_t>(part % subs) * share;
+  const int32_t row0 = entry.x < 0 ? -1 : entry.x + skip;
   const int32_t seq = entry.z;
   // Uniform exits for entries outside every sequence; an empty cache
   // (num_blocks == 0) has no row to read, and its entries store (-inf, 0).
   if (entry.y <= 0 || seq < 0 || seq >= num_seqs || row0 < 0) return;
-  const int32_t nrows = num_blocks > 0 ? min(entry.y, kEntryRows) : 0;
+  const int32_t nrows = num_blocks > 0 ? max(0, min(min(entry.y, kEntryRows) - skip, share)) : 0;
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -646,6 +675,28 @@ __global__ __launch_bounds__(kDecThreads) void attn_decode_entry_kernel(
     const int64_t qh = static_cast<int64_t>(kh) * group + g;
     emit_partial(part_acc + (part * num_q_heads + qh) * (kHeadDim / 2),
                  part_ml + part * num_q_heads + qh, a0, a1, mm, lsum, lane);
+  }
+}
+
+// One workgroup per item; a grid smaller than the items (the caller bounds
+// it by the context total it knows) goes round again.
+template <bool kWide, bool kHalf>
+__global__ __launch_bounds__(kDecThreads) void attn_decode_entry_kernel(
+    const uint16_t* __restrict__ q, int64_t q_seq_stride,
+    const uint8_t* __restrict__ key_cache, const uint8_t* __restrict__ value_cache,
+    const int32_t* __restrict__ tables, int64_t table_stride, int32_t block_size,
+    int32_t num_blocks, int32_t num_kv_heads, int32_t group, const int4* __restrict__ plan,
+    const int32_t* __restrict__ first_part, int32_t num_seqs, int32_t capacity, float scale_log2,
+    uint32_t* __restrict__ part_acc, f32x2* __restrict__ part_ml) {
+  __shared__ EntryShared sh;
+  const int32_t entries = min(((const const_i32*)first_part)[num_seqs], capacity);
+  const int32_t subs = entry_parts(entries, num_kv_heads, capacity);
+  const int64_t items = static_cast<int64_t>(entries) * subs * num_kv_heads;
+  for (int64_t item = blockIdx.x; item < items; item += gridDim.x) {
+    decode_entry<kWide, kHalf>(sh, item, subs, q, q_seq_stride, key_cache, value_cache, tables,
+                               table_stride, block_size, num_blocks, num_kv_heads, group, plan,
+                               num_seqs, scale_log2, part_acc, part_ml);
+    if (item + gridDim.x < items) __syncthreads();  // the next item reuses the LDS
   }
 }
 
@@ -1096,32 +1147,43 @@ __global__ __launch_bounds__(kDecThreads) void attn_decode_range_kernel(
   }
 }
 
-// Merges the partials of (sequence, query head) pairs, one wavefront per
-// pair and no LDS or barrier: lane i loads part i's (m + k, l 2^-k), and
-// every lane loads its two dims (one fp16 pair) of up to kReduceBatch parts
-// in the same round trip, so the merge waits for memory twice (the
-// sequence's part range, then the parts) instead of three times.  The wave
-// takes the parts' max with lane shuffles, weights and sums the parts in
-// fp32 (part i's m and l come from lane i by shuffle) and divides once.  A
-// sequence of more than kReduceBatch parts goes in batches, the running sums
-// rescaled when a later batch raises the max.
-constexpr int kReduceWaves = 4;  // pairs per workgroup
-constexpr int kReduceThreads = kReduceWaves * kWave;
-constexpr int kReduceBatch = 8;  // parts in flight per lane
+// Merges the partials of (sequence, query head) pairs, kWaves wavefronts
+// per pair.  A wave takes every kWaves-th batch of kReduceBatch parts: lane
+// i loads part i's (m + k, l 2^-k), and every lane loads its two dims (one
+// fp16 pair) of the batch's parts in the same round trip, so a batch waits
+// for memory once.  The wave takes the parts' max with lane shuffles, weights
+// and sums the parts in fp32 (part i's m and l come from lane i by shuffle),
+// the running sums rescaled when a later batch raises the max; the waves
+// merge through LDS and the first divides once.
+// One batch after another costs about 0.8 us each, so a long context among
+// few sequences, cut into a hundred parts, took 14 us with one wave per pair
+// (8 sequences of 4 kv heads, 28 query heads): a pair gets 4 or 16 waves by
+// the average number of parts (reduce_waves).
+constexpr int kReduceThreads = 4 * kWave;  // with one wave per pair: 4 pairs per workgroup
+constexpr int kReduceBatch = 8;            // parts in flight per lane
 
-template <bool kHalf>
-__global__ __launch_bounds__(kReduceThreads) void attn_decode_reduce_kernel(
+// Waves per pair.  The parts of all sequences are about `parts` in all;
+// contexts of unlike lengths give one sequence several times its share.
+constexpr int reduce_waves(int64_t parts, int64_t num_seqs) {
+  return parts > 8 * num_seqs ? 16 : parts > 2 * num_seqs ? 4 : 1;
+}
+
+template <bool kHalf, int kWaves>
+__global__ __launch_bounds__(kWaves == 1 ? kReduceThreads : kWaves* kWave) void attn_decode_reduce_kernel(
     const uint32_t* __restrict__ part_acc, const f32x2* __restrict__ part_ml,
     const int32_t* __restrict__ first_part, const int4* __restrict__ range_plan,
     int32_t num_kv_heads, int64_t capacity, int32_t num_seqs, int32_t num_q_heads,
     uint16_t* __restrict__ out, int64_t out_seq_stride) {
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int64_t pair = static_cast<int64_t>(blockIdx.x) * kReduceWaves + wave;
+  constexpr int kPairs = kWaves == 1 ? kReduceThreads / kWave : 1;  // per workgroup
+  const int64_t pair = static_cast<int64_t>(blockIdx.x) * kPairs + (kWaves == 1 ? wave : 0);
   if (pair >= static_cast<int64_t>(num_seqs) * num_q_heads) return;  // whole waves; no barrier
   const int32_t seq = static_cast<int32_t>(pair / num_q_heads);
   const int32_t qh = static_cast<int32_t>(pair % num_q_heads);
   uint16_t* const dst = out + static_cast<int64_t>(seq) * out_seq_stride + qh * kHeadDim + 2 * lane;
+  int64_t p0 = max(0, first_part[seq]);
+  int64_t p1 = first_part[seq + 1];
   // A range plan built for another sequence or kv-head count: the range
   // kernel wrote no partial, so the workspace holds stale values.  Every
   // output becomes NaN instead.
@@ -1129,16 +1191,22 @@ __global__ __launch_bounds__(kReduceThreads) void attn_decode_reduce_kernel(
     const const_i32* const header = (const const_i32*)range_plan;
     if (header[2] != num_seqs || header[3] != num_kv_heads) {
       const uint16_t nan = kHalf ? 0x7E00u : 0x7FC0u;
-      *reinterpret_cast<uint32_t*>(dst) = static_cast<uint32_t>(nan) | (static_cast<uint32_t>(nan) << 16);
-      return;
+      if (kWaves == 1 || wave == 0) {
+        *reinterpret_cast<uint32_t*>(dst) = static_cast<uint32_t>(nan) | (static_cast<uint32_t>(nan) << 16);
+      }
+      return;  // every wave of the workgroup
     }
+  } else {
+    const int32_t entries = min(static_cast<int64_t>(first_part[num_seqs]), capacity);
+    const int32_t subs = entry_parts(entries, num_kv_heads, capacity);
+    p0 *= subs;
+    p1 *= subs;
   }
-  const int64_t p0 = max(0, first_part[seq]);
-  const int64_t p1 = min(capacity, static_cast<int64_t>(first_part[seq + 1]));
+  p1 = min(capacity, p1);
 
   float run_max = -INFINITY;  // max of the parts merged so far
   float ax = 0.f, ay = 0.f, lsum = 0.f;
-  for (int64_t b = p0; b < p1; b += kReduceBatch) {
+  for (int64_t b = p0 + (kWaves == 1 ? 0 : wave * kReduceBatch); b < p1; b += kWaves * kReduceBatch) {
     const int n = static_cast<int>(min(static_cast<int64_t>(kReduceBatch), p1 - b));
     f32x2 ml = {-INFINITY, 0.f};  // lane i < n: part b + i's (m + k, l 2^-k)
     if (lane < n) ml = part_ml[(b + lane) * num_q_heads + qh];
@@ -1169,10 +1237,42 @@ __global__ __launch_bounds__(kReduceThreads) void attn_decode_reduce_kernel(
     }
     run_max = new_max;
   }
+  if constexpr (kWaves > 1) {
+    __shared__ f32x2 s_sums[kWaves][kWave];
+    __shared__ f32x2 s_ml[kWaves];
+    s_sums[wave][lane] = f32x2{ax, ay};
+    if (lane == 0) s_ml[wave] = f32x2{run_max, lsum};
+    __syncthreads();
+    if (wave != 0) return;
+    float top = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) top = fmaxf(top, s_ml[w].x);
+    ax = 0.f;
+    ay = 0.f;
+    lsum = 0.f;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      const f32x2 ml = s_ml[w];
+      const f32x2 v = s_sums[w][lane];
+      const float f = ml.x == -INFINITY ? 0.f : exp2_fast(ml.x - top);
+      ax = fmaf(v.x, f, ax);
+      ay = fmaf(v.y, f, ay);
+      lsum = fmaf(ml.y, f, lsum);
+    }
+  }
   const bool any = lsum > 0.f;
   const uint32_t packed = static_cast<uint32_t>(from_f32<kHalf>(any ? ax / lsum : 0.f)) |
                           (static_cast<uint32_t>(from_f32<kHalf>(any ? ay / lsum : 0.f)) << 16);
   *reinterpret_cast<uint32_t*>(dst) = packed;
+}
+
+using ReduceKernel = void (*)(const uint32_t*, const f32x2*, const int32_t*, const int4*, int32_t,
+                              int64_t, int32_t, int32_t, uint16_t*, int64_t);
+template <bool kHalf>
+ReduceKernel reduce_kernel_for(int waves) {
+  return waves == 16  ? attn_decode_reduce_kernel<kHalf, 16>
+         : waves == 4 ? attn_decode_reduce_kernel<kHalf, 4>
+                      : attn_decode_reduce_kernel<kHalf, 1>;
 }
 
 using RangeKernel = void (*)(const uint16_t*, int64_t, const uint8_t*, const uint8_t*,
@@ -1181,7 +1281,8 @@ using RangeKernel = void (*)(const uint16_t*, int64_t, const uint8_t*, const uin
                               f32x2*);
 using EntryKernel = void (*)(const uint16_t*, int64_t, const uint8_t*, const uint8_t*,
                               const int32_t*, int64_t, int32_t, int32_t, int32_t, int32_t,
-                              const int4*, int32_t, float, uint32_t*, f32x2*);
+                              const int4*, const int32_t*, int32_t, int32_t, float, uint32_t*,
+                              f32x2*);
 
 RangeKernel range_kernel_for(bool wide, bool half) {
   if (wide) return half ? attn_decode_range_kernel<true, true> : attn_decode_range_kernel<true, false>;
@@ -1268,6 +1369,19 @@ extern "C" int nkv_paged_attention_decode(
     const int32_t* first_part, int64_t num_seqs, int64_t num_kv_heads, int64_t num_q_heads,
     int64_t head_dim, int64_t block_size, int64_t num_blocks, float scale, int32_t dtype,
     void* workspace, int64_t workspace_bytes, void* out, int64_t out_seq_stride, void* stream) {
+  return nkv_paged_attention_decode_total(
+      q, q_seq_stride, key_cache, value_cache, block_tables, table_stride, plan, capacity, first_part,
+      num_seqs, num_kv_heads, num_q_heads, head_dim, block_size, num_blocks, scale, dtype, workspace,
+      workspace_bytes, out, out_seq_stride, -1, stream);
+}
+
+extern "C" int nkv_paged_attention_decode_total(
+    const void* q, int64_t q_seq_stride, const void* key_cache, const void* value_cache,
+    const int32_t* block_tables, int64_t table_stride, const void* plan, int64_t capacity,
+    const int32_t* first_part, int64_t num_seqs, int64_t num_kv_heads, int64_t num_q_heads,
+    int64_t head_dim, int64_t block_size, int64_t num_blocks, float scale, int32_t dtype,
+    void* workspace, int64_t workspace_bytes, void* out, int64_t out_seq_stride,
+    int64_t total_tokens, void* stream) {
   using namespace nkv;
   if (dtype != NKV_DTYPE_BFLOAT16 && dtype != NKV_DTYPE_FLOAT16) {
     return nkv_fail(NKV_E_INVALID,
@@ -1342,14 +1456,23 @@ extern "C" int nkv_paged_attention_decode(
     if (capacity * num_kv_heads > INT32_MAX) {
       return nkv_fail(NKV_E_INVALID, "nkv_paged_attention_decode: plan too long for the grid");
     }
-    entry_kernel_for(wide, half)<<<dim3(static_cast<unsigned>(capacity * num_kv_heads)),
+    // Workgroups for every entry the context total allows, or for the parts
+    // of cut entries.  (The plan's capacity also holds the range split's
+    // partials: 8,232 workgroups for the 56 items of one 5,003-row sequence.)
+    int64_t most = capacity;
+    if (total_tokens >= 0) {
+      most = std::max(entry_plan_capacity(total_tokens, num_seqs, block_size),
+                      kHalvesTarget / num_kv_heads + 1);
+      most = std::min(most, capacity);
+    }
+    entry_kernel_for(wide, half)<<<dim3(static_cast<unsigned>(most * num_kv_heads)),
                                    dim3(kDecThreads), 0, s>>>(
         static_cast<const uint16_t*>(q), q_seq_stride, static_cast<const uint8_t*>(key_cache),
         static_cast<const uint8_t*>(value_cache), block_tables, table_stride,
         static_cast<int32_t>(block_size), static_cast<int32_t>(num_blocks),
         static_cast<int32_t>(num_kv_heads), static_cast<int32_t>(group),
-        static_cast<const int4*>(plan), static_cast<int32_t>(num_seqs), scale_log2, part_acc,
-        part_ml);
+        static_cast<const int4*>(plan), first_part, static_cast<int32_t>(num_seqs),
+        static_cast<int32_t>(capacity), scale_log2, part_acc, part_ml);
   } else if (!entries) {
     const int64_t waves = workers_per_head(num_kv_heads) * num_kv_heads;
     range_kernel_for(wide, half)<<<dim3(static_cast<unsigned>((waves + kDecWaves - 1) / kDecWaves)),
@@ -1362,20 +1485,17 @@ extern "C" int nkv_paged_attention_decode(
         static_cast<int32_t>(capacity), scale_log2, part_acc, part_ml);
   }
   if (int rc = nkv_check_launch("nkv_paged_attention_decode (partials)")) return rc;
-  // one wavefront per (sequence, query head) pair, kReduceWaves pairs per workgroup
-  const int64_t pairs = num_seqs * num_q_heads;
   const int4* const range_plan = entries ? nullptr : static_cast<const int4*>(plan);
-  const dim3 reduce_grid(static_cast<unsigned>((pairs + kReduceWaves - 1) / kReduceWaves));
-  if (half) {
-    attn_decode_reduce_kernel<true><<<reduce_grid, dim3(kReduceThreads), 0, s>>>(
-        part_acc, part_ml, first_part, range_plan, static_cast<int32_t>(num_kv_heads), capacity,
-        static_cast<int32_t>(num_seqs), static_cast<int32_t>(num_q_heads),
-        static_cast<uint16_t*>(out), out_seq_stride);
-  } else {
-    attn_decode_reduce_kernel<false><<<reduce_grid, dim3(kReduceThreads), 0, s>>>(
-        part_acc, part_ml, first_part, range_plan, static_cast<int32_t>(num_kv_heads), capacity,
-        static_cast<int32_t>(num_seqs), static_cast<int32_t>(num_q_heads),
-        static_cast<uint16_t*>(out), out_seq_stride);
-  }
+  // Parts of all sequences at most (long contexts of the entry split aside).
+  const int64_t parts = entries ? kPartsTarget / num_kv_heads : workers_per_head(num_kv_heads);
+  const int waves = reduce_waves(parts, num_seqs);
+  const int64_t pairs = num_seqs * num_q_heads;
+  const int64_t per_group = waves == 1 ? kReduceThreads / kWave : 1;
+  const ReduceKernel reduce = half ? reduce_kernel_for<true>(waves) : reduce_kernel_for<false>(waves);
+  reduce<<<dim3(static_cast<unsigned>((pairs + per_group - 1) / per_group)),
+           dim3(waves == 1 ? kReduceThreads : waves * kWave), 0, s>>>(
+      part_acc, part_ml, first_part, range_plan, static_cast<int32_t>(num_kv_heads), capacity,
+      static_cast<int32_t>(num_seqs), static_cast<int32_t>(num_q_heads),
+      static_cast<uint16_t*>(out), out_seq_stride);
   return nkv_check_launch("nkv_paged_attention_decode (reduce)");
 }

@@ -119,6 +119,14 @@ SIGNATURES: dict[str, tuple[object, tuple[object, ...]]] = {
             c_ptr,
         ),
     ),
+    "nkv_paged_attention_decode_total": (
+        ctypes.c_int,
+        (
+            c_ptr, c_i64, c_ptr, c_ptr, c_ptr, c_i64, c_ptr, c_i64, c_ptr, c_i64, c_i64,
+            c_i64, c_i64, c_i64, c_i64, ctypes.c_float, c_i32, c_ptr, c_i64, c_ptr, c_i64,
+            c_i64, c_ptr,
+        ),
+    ),
     "nkv_prefill_tile_tokens": (c_i64, (c_i64,)),
     "nkv_prefill_plan_capacity": (c_i64, (c_i64, c_i64, c_i64)),
     "nkv_build_prefill_plan": (ctypes.c_int, (c_ptr, c_ptr, c_i64, c_i64, c_ptr, c_i64, c_ptr)),

@@ -333,7 +333,8 @@ class HIPPagedKVBackend:
         if out is None:
             out = torch.empty_like(q)
         ops.paged_attention_decode(
-            q, key_cache, value_cache, block_tables, plan[0], plan[1], float(softmax_scale), out
+            q, key_cache, value_cache, block_tables, plan[0], plan[1], float(softmax_scale), out,
+            int(total_tokens),
         )
         return out
 

@@ -25,7 +25,7 @@ too, paged_kv_cuda.cu:168-171).  Additive ops, with no reference schema:
     paged_attention_decode(Tensor q, Tensor key_cache, Tensor value_cache,
                            Tensor block_tables, Tensor plan,
                            Tensor first_part, float scale,
-                           Tensor(a!) out) -> ()
+                           Tensor(a!) out, int total_tokens=-1) -> ()
     build_store_gather_plan(Tensor block_tables, Tensor cu_seqlens_q,
                             Tensor cu_seqlens_k, int num_tokens,
                             int total_tokens, int num_blocks, int block_size,
@@ -62,7 +62,7 @@ SCHEMAS = {
     "int block_size, int num_kv_heads) -> (Tensor, Tensor)",
     "paged_attention_decode": "paged_attention_decode(Tensor q, Tensor key_cache, "
     "Tensor value_cache, Tensor block_tables, Tensor plan, Tensor first_part, float scale, "
-    "Tensor(a!) out) -> ()",
+    "Tensor(a!) out, int total_tokens=-1) -> ()",
     "build_store_gather_plan": "build_store_gather_plan(Tensor block_tables, "
     "Tensor cu_seqlens_q, Tensor cu_seqlens_k, int num_tokens, int total_tokens, "
     "int num_blocks, int block_size, int row_elems, ScalarType dtype) -> Tensor",
@@ -419,7 +419,7 @@ def _build_attention_plan_impl(cu_seqlens_k, total_tokens: int, block_size: int,
 
 
 def _paged_attention_decode_impl(q, key_cache, value_cache, block_tables, plan, first_part,
-                                 scale: float, out) -> None:
+                                 scale: float, out, total_tokens: int = -1) -> None:
     device = _require_device(
         "paged KV HIP attention", q, key_cache, value_cache, block_tables, plan, first_part, out
     )
@@ -443,13 +443,13 @@ def _paged_attention_decode_impl(q, key_cache, value_cache, block_tables, plan, 
     capacity = plan.shape[0]
     nbytes = int(library.nkv_attention_workspace_bytes(capacity, q.shape[1], head_dim))
     workspace = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=device)
-    status = library.nkv_paged_attention_decode(
+    status = library.nkv_paged_attention_decode_total(
         q.data_ptr(), q.stride(0), key_cache.data_ptr(), value_cache.data_ptr(),
         block_tables.data_ptr(), block_tables.shape[1],
         plan.data_ptr() if capacity else None, capacity, first_part.data_ptr(), q.shape[0],
         num_kv_heads, q.shape[1], head_dim, block_size, num_blocks, float(scale),
         DTYPE_CODES[q.dtype], workspace.data_ptr(), workspace.numel(), out.data_ptr(),
-        out.stride(0), _stream(device),
+        out.stride(0), total_tokens, _stream(device),
     )
     _lib.check(status, "nanovllm_paged_kv::paged_attention_decode")
 

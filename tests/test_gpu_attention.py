@@ -538,3 +538,30 @@ def test_decode_step_layer_full_size(backend, gpu_device, hq):
     ref = reference(dict(q=q.float().cpu().numpy(), kc=hk, vc=hv, tables=ctables,
                          lens=wl.num_tokens), 1 / math.sqrt(128))
     check_close(out, ref, f"decode step layer, {hq} query heads")
+
+
+@pytest.mark.parametrize("hkv,g,lens", [
+    (8, 2, [5003]),                       # one long context: entries in 16 parts, 16 waves merge
+    (8, 4, [1, 17, 768, 769, 0, 95]),     # parts of every fill, empty parts, an empty context
+    (16, 1, [2000] * 20),                 # halves
+    (8, 2, [3000] * 80),                  # whole entries, one wave merges
+    (4, 7, [16000, 3, 40]),               # range split: one context in most of the parts
+    (1, 8, [9000]),                       # 563 parts of one context
+    (2, 16, [700, 0, 33, 1200] * 40),     # range split, few parts per context
+])
+def test_cut_entries_and_wide_merges(backend, gpu_device, hkv, g, lens):
+    """Launches whose entries are cut into parts and merges by 1, 4 and 16
+    wavefronts per (sequence, head): against the oracle, and equal whether or
+    not the launch knows the context total (which bounds its grid)."""
+    from nanokv.paged_kv import ops
+
+    dev, host, total = build_case(gpu_device, hkv, g, 16, lens, seed=len(lens) + hkv)
+    plan = backend.build_attention_plan(dev["kc"], dev["cu"], total)
+    out = backend.paged_attention_decode(dev["q"], dev["kc"], dev["vc"], dev["tables"], dev["cu"],
+                                         total, 0.1, plan=plan)
+    check_close(out, reference(host, 0.1), f"hkv={hkv} g={g}")
+    for known in (-1, 0):  # unknown; an understatement makes each workgroup go round more often
+        again = torch.full_like(out, float("nan"))
+        ops.paged_attention_decode(dev["q"], dev["kc"], dev["vc"], dev["tables"], plan[0], plan[1],
+                                   0.1, again, known)
+        assert torch.equal(out, again), known
