@@ -385,6 +385,12 @@ int nkv_build_attention_plan(const int32_t* cu_seqlens_k, int64_t num_seqs,
                              int64_t block_size, int64_t num_kv_heads,
                              void* plan, int64_t capacity,
                              int32_t* first_part, void* stream);
+/* The same plan from the context lengths themselves, context_lens[num_seqs]. */
+int nkv_build_attention_plan_lengths(const int32_t* context_lens,
+                                     int64_t num_seqs, int64_t block_size,
+                                     int64_t num_kv_heads, void* plan,
+                                     int64_t capacity, int32_t* first_part,
+                                     void* stream);
 int nkv_paged_attention_decode(const void* q, int64_t q_seq_stride,
                                const void* key_cache, const void* value_cache,
                                const int32_t* block_tables, int64_t table_stride,

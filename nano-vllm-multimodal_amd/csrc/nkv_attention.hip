@@ -230,11 +230,20 @@ int64_t entry_plan_capacity(int64_t total_tokens, int64_t num_seqs, int64_t bloc
   return (total_tokens + rows - 1) / rows + num_seqs;
 }
 
+// A sequence's length: from its offsets, or given as it is.
+struct Lengths {
+  const int32_t* values;
+  bool offsets;
+  __device__ __forceinline__ int32_t operator()(int32_t i) const {
+    return offsets ? values[i + 1] - values[i] : values[i];
+  }
+};
+
 // One workgroup: the unit offsets of the sequences by an LDS scan, then the
 // partial counts (a second pass over the same runs, straight to
 // first_part), then one record per worker by binary search.
 __global__ __launch_bounds__(kPlanThreads) void attn_range_plan_kernel(
-    const int32_t* __restrict__ cu_seqlens, int32_t num_seqs, int32_t num_kv_heads,
+    Lengths length_of, int32_t num_seqs, int32_t num_kv_heads,
     int4* __restrict__ plan, int32_t* __restrict__ first_part) {
   extern __shared__ int32_t s_mem[];
   int32_t* s_unit = s_mem;                // [num_seqs + 1] first unit of each sequence
@@ -242,7 +251,7 @@ __global__ __launch_bounds__(kPlanThreads) void attn_range_plan_kernel(
   lds_exclusive_scan<kPlanThreads>(
       num_seqs,
       [&](int32_t i) {
-        const int32_t len = cu_seqlens[i + 1] - cu_seqlens[i];
+        const int32_t len = length_of(i);
         return len > 0 ? (len + kDecKeys - 1) / kDecKeys + kDecSegCost : 0;
       },
       s_unit, s_tmp);
@@ -268,7 +277,7 @@ __global__ __launch_bounds__(kPlanThreads) void attn_range_plan_kernel(
   for (int32_t i = begin; i < end; ++i) {
     first_part[i] = base;
     base += parts_of(i);
-    lens[i] = cu_seqlens[i + 1] - cu_seqlens[i];
+    lens[i] = length_of(i);
     vstart[i] = s_unit[i] + kDecSegCost;
   }
   if (threadIdx.x == 0) {
@@ -311,7 +320,7 @@ __global__ __launch_bounds__(kPlanThreads) void attn_range_plan_kernel(
 // Every workgroup rescans the per-sequence entry counts in LDS, so one
 // launch builds the whole plan.  Entries past the total get rows = 0.
 __global__ __launch_bounds__(kPlanThreads) void attn_entry_plan_kernel(
-    const int32_t* __restrict__ cu_seqlens, int32_t num_seqs, int32_t entry_rows,
+    Lengths length_of, int32_t num_seqs, int32_t entry_rows,
     int4* __restrict__ plan, int64_t capacity, int32_t* __restrict__ first_part) {
   extern __shared__ int32_t s_mem[];
   int32_t* s_first = s_mem;               // [num_seqs + 1]
@@ -319,7 +328,7 @@ __global__ __launch_bounds__(kPlanThreads) void attn_entry_plan_kernel(
   lds_exclusive_scan<kPlanThreads>(
       num_seqs,
       [&](int32_t i) {
-        const int32_t len = cu_seqlens[i + 1] - cu_seqlens[i];
+        const int32_t len = length_of(i);
         return len > 0 ? (len + entry_rows - 1) / entry_rows : 0;
       },
       s_first, s_tmp);
@@ -334,7 +343,7 @@ __global__ __launch_bounds__(kPlanThreads) void attn_entry_plan_kernel(
     if (e < total) {
       const int32_t i = owner_of(s_first, num_seqs, static_cast<int32_t>(e));
       const int32_t row0 = (static_cast<int32_t>(e) - s_first[i]) * entry_rows;
-      const int32_t len = cu_seqlens[i + 1] - cu_seqlens[i];
+      const int32_t len = length_of(i);
       entry = make_int4(row0, min(entry_rows, len - row0), i, 0);
     }
     plan[e] = entry;
@@ -1317,10 +1326,11 @@ extern "C" int64_t nkv_attention_workspace_bytes(int64_t capacity, int64_t num_q
   return capacity * num_q_heads * (head_dim * 2 + 8);
 }
 
-extern "C" int nkv_build_attention_plan(const int32_t* cu_seqlens_k, int64_t num_seqs,
-                                        int64_t block_size, int64_t num_kv_heads, void* plan,
-                                        int64_t capacity, int32_t* first_part, void* stream) {
-  using namespace nkv;
+namespace nkv {
+namespace {
+
+int build_attention_plan(Lengths lengths, int64_t num_seqs, int64_t block_size, int64_t num_kv_heads,
+                         void* plan, int64_t capacity, int32_t* first_part, void* stream) {
   if (num_seqs < 0 || num_seqs > NKV_MAX_PLAN_SEQS) {
     return nkv_fail(NKV_E_INVALID, "nkv_build_attention_plan: num_seqs=%lld outside [0, %d]",
                     static_cast<long long>(num_seqs), NKV_MAX_PLAN_SEQS);
@@ -1338,7 +1348,7 @@ extern "C" int nkv_build_attention_plan(const int32_t* cu_seqlens_k, int64_t num
                     static_cast<long long>(range_plan_capacity(num_seqs)),
                     static_cast<long long>(num_seqs));
   }
-  if (!first_part || (num_seqs > 0 && !cu_seqlens_k) || ((capacity > 0 || !entries) && !plan)) {
+  if (!first_part || (num_seqs > 0 && !lengths.values) || ((capacity > 0 || !entries) && !plan)) {
     return nkv_fail(NKV_E_INVALID, "nkv_build_attention_plan: null pointer");
   }
   if (reinterpret_cast<uint64_t>(plan) % 16 != 0) {
@@ -1352,15 +1362,34 @@ extern "C" int nkv_build_attention_plan(const int32_t* cu_seqlens_k, int64_t num
     // too short for the lengths is refused by the caller, who knows them.
     const int64_t blocks = capacity > 0 ? (capacity + kPlanThreads - 1) / kPlanThreads : 1;
     attn_entry_plan_kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(kPlanThreads), lds, s>>>(
-        cu_seqlens_k, static_cast<int32_t>(num_seqs),
+        lengths, static_cast<int32_t>(num_seqs),
         static_cast<int32_t>(attention_entry_rows(block_size)), static_cast<int4*>(plan),
         capacity, first_part);
   } else {
     attn_range_plan_kernel<<<dim3(1), dim3(kPlanThreads), lds, s>>>(
-        cu_seqlens_k, static_cast<int32_t>(num_seqs), static_cast<int32_t>(num_kv_heads),
+        lengths, static_cast<int32_t>(num_seqs), static_cast<int32_t>(num_kv_heads),
         static_cast<int4*>(plan), first_part);
   }
   return nkv_check_launch("nkv_build_attention_plan");
+}
+
+}  // namespace
+}  // namespace nkv
+
+extern "C" int nkv_build_attention_plan(const int32_t* cu_seqlens_k, int64_t num_seqs,
+                                        int64_t block_size, int64_t num_kv_heads, void* plan,
+                                        int64_t capacity, int32_t* first_part, void* stream) {
+  return nkv::build_attention_plan(nkv::Lengths{cu_seqlens_k, true}, num_seqs, block_size, num_kv_heads,
+                                   plan, capacity, first_part, stream);
+}
+
+// The lengths themselves, as a captured step holds them: offsets for them
+// were a fill and a scan per layer, 4.5 us each in the graph.
+extern "C" int nkv_build_attention_plan_lengths(const int32_t* context_lens, int64_t num_seqs,
+                                        int64_t block_size, int64_t num_kv_heads, void* plan,
+                                        int64_t capacity, int32_t* first_part, void* stream) {
+  return nkv::build_attention_plan(nkv::Lengths{context_lens, false}, num_seqs, block_size, num_kv_heads,
+                                   plan, capacity, first_part, stream);
 }
 
 extern "C" int nkv_paged_attention_decode(

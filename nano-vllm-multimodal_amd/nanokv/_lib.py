@@ -111,6 +111,10 @@ SIGNATURES: dict[str, tuple[object, tuple[object, ...]]] = {
         ctypes.c_int,
         (c_ptr, c_i64, c_i64, c_i64, c_ptr, c_i64, c_ptr, c_ptr),
     ),
+    "nkv_build_attention_plan_lengths": (
+        ctypes.c_int,
+        (c_ptr, c_i64, c_i64, c_i64, c_ptr, c_i64, c_ptr, c_ptr),
+    ),
     "nkv_paged_attention_decode": (
         ctypes.c_int,
         (

@@ -287,6 +287,21 @@ class HIPPagedKVBackend:
         return AttentionPlan(plan, first_part,
                              (int(total_tokens), int(cu_seqlens_k.numel()) - 1, int(cache.shape[2])))
 
+    def build_attention_plan_from_lengths(
+        self,
+        cache: torch.Tensor,
+        context_lens: torch.Tensor,
+        total_tokens: int,
+    ) -> "AttentionPlan":
+        """The same plan from the context lengths themselves (contiguous 1-D
+        int32), for callers without their offsets; ``total_tokens`` may
+        overstate their sum, as under graph capture."""
+        self._load()
+        plan, first_part = ops.attention_plan_from_lengths(context_lens, total_tokens, cache.shape[1],
+                                                           cache.shape[2])
+        return AttentionPlan(plan, first_part,
+                             (int(total_tokens), int(context_lens.numel()), int(cache.shape[2])))
+
     def paged_attention_decode(
         self,
         q: torch.Tensor,

@@ -399,13 +399,26 @@ def _build_attention_plan_impl(cu_seqlens_k, total_tokens: int, block_size: int,
     device = _require_device("paged KV HIP attention plan", cu_seqlens_k)
     if cu_seqlens_k.dtype != torch.int32 or cu_seqlens_k.ndim != 1 or not cu_seqlens_k.is_contiguous():
         raise ValueError("cu_seqlens_k must be a contiguous 1-D int32 tensor")
-    num_seqs = cu_seqlens_k.numel() - 1
+    return _attention_plan("nkv_build_attention_plan", device, cu_seqlens_k, cu_seqlens_k.numel() - 1,
+                           total_tokens, block_size, num_kv_heads)
+
+
+def attention_plan_from_lengths(context_lens, total_tokens: int, block_size: int, num_kv_heads: int):
+    """(plan, first_part) as build_attention_plan gives them, from the
+    context lengths themselves (contiguous 1-D int32)."""
+    device = _require_device("paged KV HIP attention plan", context_lens)
+    return _attention_plan("nkv_build_attention_plan_lengths", device, context_lens,
+                           context_lens.numel(), total_tokens, block_size, num_kv_heads)
+
+
+def _attention_plan(builder: str, device, lengths, num_seqs: int, total_tokens: int, block_size: int,
+                    num_kv_heads: int):
     library = _lib.load_library()
     capacity = int(library.nkv_attention_plan_capacity(total_tokens, num_seqs, block_size))
     plan = torch.empty((capacity, 4), dtype=torch.int32, device=device)
     first_part = torch.empty(num_seqs + 1, dtype=torch.int32, device=device)
-    status = library.nkv_build_attention_plan(
-        cu_seqlens_k.data_ptr(),
+    status = getattr(library, builder)(
+        lengths.data_ptr(),
         num_seqs,
         block_size,
         num_kv_heads,

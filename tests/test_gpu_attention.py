@@ -565,3 +565,19 @@ def test_cut_entries_and_wide_merges(backend, gpu_device, hkv, g, lens):
         ops.paged_attention_decode(dev["q"], dev["kc"], dev["vc"], dev["tables"], plan[0], plan[1],
                                    0.1, again, known)
         assert torch.equal(out, again), known
+
+
+@pytest.mark.parametrize("hkv", [2, 8])
+@pytest.mark.parametrize("lens", [[0], [5], [769, 0, 31, 768], list(range(0, 3000, 7))])
+def test_plan_from_lengths_equals_plan_from_offsets(backend, gpu_device, hkv, lens):
+    """Both plan builders write the same plan and first parts."""
+    cache = torch.empty((1, 16, hkv, 128), dtype=torch.bfloat16, device=gpu_device)
+    given = torch.tensor(lens, dtype=torch.int32, device=gpu_device)
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int32, device=gpu_device)
+    total = sum(lens)
+    one = backend.build_attention_plan(cache, cu, total)
+    other = backend.build_attention_plan_from_lengths(cache, given, total)
+    assert other.lengths == one.lengths
+    assert torch.equal(one[1], other[1])
+    used = int(one[1][-1]) if hkv >= 8 else 1 + 1024  # entries, or the header and the workers' records
+    assert torch.equal(one[0][:used], other[0][:used])
