@@ -1,4 +1,4 @@
-// Per-call host path of the hip backend's store and gather.
+// Per-call host path of the hip backend's store, gather and attention.
 //
 // The reference's SDPA decode calls its backend's gather twice per request
 // per layer (nanovllm/layers/attention.py:284-300) and its store once per
@@ -18,6 +18,7 @@
 // caller's current stream, passed in as a hipStream_t integer.
 #include <torch/extension.h>
 
+#include <algorithm>
 #include <cctype>
 #include <cstdint>
 #include <cstdlib>
@@ -195,6 +196,192 @@ at::Tensor gather(const at::Tensor& cache, const at::Tensor& table, int64_t sequ
   return out;
 }
 
+// ------------------------------------------------------------- attention
+//
+// One layer's attention call, whole, for the calls an engine makes: every
+// tensor as the kernels take it.  A call that any check of the Python path
+// would refuse, convert or look into returns None instead, and the Python
+// path serves it (or raises), so nothing is decided twice.  Per call the
+// Python checks, allocations and ctypes conversions were 17-20 us of host
+// time, more than the kernels of a short context take.
+using PlanCapacityFn = int64_t (*)(int64_t, int64_t, int64_t);
+using WorkspaceFn = int64_t (*)(int64_t, int64_t, int64_t);
+using DecodeFn = decltype(&nkv_paged_attention_decode_total);
+using PrefillPlanFn = decltype(&nkv_build_prefill_plan);
+using PrefillFn = decltype(&nkv_paged_attention_prefill_split);
+using VarlenFn = decltype(&nkv_varlen_attention_prefill);
+
+PlanCapacityFn g_decode_capacity = nullptr;
+WorkspaceFn g_decode_workspace = nullptr;
+DecodeFn g_decode = nullptr;
+PlanCapacityFn g_prefill_capacity = nullptr;
+PrefillPlanFn g_prefill_plan = nullptr;
+WorkspaceFn g_prefill_workspace = nullptr;
+PrefillFn g_prefill = nullptr;
+VarlenFn g_varlen = nullptr;
+
+constexpr int64_t kDim = 128;
+
+bool on(const at::Tensor& t, const at::Device& device) { return t.device() == device; }
+bool int32_vector(const at::Tensor& t, const at::Device& device) {
+  return t.scalar_type() == at::kInt && t.dim() == 1 && t.is_contiguous() && on(t, device);
+}
+bool int32_matrix(const at::Tensor& t, const at::Device& device) {
+  return t.scalar_type() == at::kInt && t.dim() == 2 && t.is_contiguous() && on(t, device);
+}
+bool half_type(at::ScalarType type) { return type == at::kHalf || type == at::kBFloat16; }
+// [rows, heads, 128] with each row's heads in one run.
+bool head_rows(const at::Tensor& t, at::ScalarType type, const at::Device& device) {
+  return t.dim() == 3 && t.scalar_type() == type && on(t, device) && t.size(2) == kDim &&
+         t.stride(2) == 1 && t.stride(1) == kDim;
+}
+bool caches(const at::Tensor& k, const at::Tensor& v, at::ScalarType type, const at::Device& device) {
+  return k.dim() == 4 && k.sizes() == v.sizes() && k.scalar_type() == type && v.scalar_type() == type &&
+         on(k, device) && on(v, device) && k.is_contiguous() && v.is_contiguous() && k.size(2) > 0 &&
+         k.size(3) == kDim;
+}
+// The output to write: the caller's, or a new one; undefined when the
+// caller's is not one the kernels write as it is.
+at::Tensor output_for(const at::Tensor& q, const c10::optional<at::Tensor>& out) {
+  if (!out.has_value()) return at::empty_like(q);
+  if (out->sizes() != q.sizes() || !head_rows(*out, q.scalar_type(), q.device())) return {};
+  return *out;
+}
+at::Tensor bytes_on(int64_t bytes, const at::Tensor& like) {
+  return at::empty({bytes}, like.options().dtype(at::kByte));
+}
+void* data_or_null(const at::Tensor& t) { return t.size(0) > 0 ? t.data_ptr() : nullptr; }
+
+py::object decode(const at::Tensor& q, const at::Tensor& key_cache, const at::Tensor& value_cache,
+                  const at::Tensor& tables, const at::Tensor& cu_seqlens_k, const at::Tensor& plan,
+                  const at::Tensor& first_part, int64_t total_tokens, double scale,
+                  const c10::optional<at::Tensor>& out_in, int64_t stream) {
+  const at::Device device = q.device();
+  const at::ScalarType type = q.scalar_type();
+  if (g_decode == nullptr || !q.is_cuda() || !half_type(type) || !head_rows(q, type, device) ||
+      !caches(key_cache, value_cache, type, device) || !int32_matrix(tables, device) ||
+      !int32_vector(cu_seqlens_k, device) || !int32_matrix(plan, device) ||
+      !int32_vector(first_part, device) || total_tokens < 0 || index_values_checked(cu_seqlens_k)) {
+    return py::none();
+  }
+  const int64_t seqs = q.size(0);
+  if (seqs == 0 || tables.size(0) != seqs || cu_seqlens_k.size(0) != seqs + 1 ||
+      first_part.size(0) != seqs + 1 || plan.size(1) != 4 ||
+      plan.size(0) < g_decode_capacity(total_tokens, seqs, key_cache.size(1))) {
+    return py::none();
+  }
+  const at::Tensor out = output_for(q, out_in);
+  if (!out.defined()) return py::none();
+  const int64_t capacity = plan.size(0);
+  const int64_t need = std::max<int64_t>(g_decode_workspace(capacity, q.size(1), kDim), 16);
+  const at::Tensor workspace = bytes_on(need, q);
+  check_status(g_decode(q.data_ptr(), q.stride(0), key_cache.data_ptr(), value_cache.data_ptr(),
+                        tables.data_ptr<int32_t>(), tables.size(1), data_or_null(plan), capacity,
+                        first_part.data_ptr<int32_t>(), seqs, key_cache.size(2), q.size(1), kDim,
+                        key_cache.size(1), key_cache.size(0), static_cast<float>(scale),
+                        dtype_code(type), workspace.data_ptr(), need, out.data_ptr(), out.stride(0),
+                        total_tokens, reinterpret_cast<void*>(stream)),
+               "nanovllm_paged_kv::paged_attention_decode");
+  return py::cast(out);
+}
+
+// A prefill plan for these offsets, or undefined where the head layout has none.
+at::Tensor prefill_plan(const at::Tensor& q, int64_t kv_heads, const at::Tensor& cu_q,
+                        const at::Tensor& cu_k, int64_t stream) {
+  const int64_t seqs = cu_q.size(0) - 1, group = q.size(1) / kv_heads;
+  const int64_t capacity = g_prefill_capacity(q.size(0), seqs, group);
+  if (capacity == 0) return {};
+  const at::Tensor plan = at::empty({capacity, 4}, cu_q.options());
+  check_status(g_prefill_plan(cu_q.data_ptr<int32_t>(), cu_k.data_ptr<int32_t>(), seqs, group,
+                              plan.data_ptr(), capacity, reinterpret_cast<void*>(stream)),
+               "nanovllm_paged_kv::build_prefill_plan");
+  return plan;
+}
+
+py::object prefill(const at::Tensor& q, const at::Tensor& key_cache, const at::Tensor& value_cache,
+                   const at::Tensor& tables, const at::Tensor& cu_q, const at::Tensor& cu_k,
+                   const c10::optional<at::Tensor>& plan_in, double scale,
+                   const c10::optional<at::Tensor>& out_in, int64_t stream) {
+  const at::Device device = q.device();
+  const at::ScalarType type = q.scalar_type();
+  if (g_prefill == nullptr || !q.is_cuda() || !half_type(type) || !head_rows(q, type, device) ||
+      !caches(key_cache, value_cache, type, device) || !int32_matrix(tables, device) ||
+      !int32_vector(cu_q, device) || !int32_vector(cu_k, device) || cu_q.size(0) != cu_k.size(0) ||
+      cu_q.size(0) < 2 || tables.size(0) != cu_q.size(0) - 1 || index_values_checked(cu_k)) {
+    return py::none();
+  }
+  const int64_t seqs = cu_q.size(0) - 1, kv_heads = key_cache.size(2);
+  if (plan_in.has_value() &&
+      (!int32_matrix(*plan_in, device) || plan_in->size(1) != 4 || q.size(1) % kv_heads != 0 ||
+       plan_in->size(0) < g_prefill_capacity(q.size(0), seqs, q.size(1) / kv_heads))) {
+    return py::none();
+  }
+  const at::Tensor out = output_for(q, out_in);
+  if (!out.defined()) return py::none();
+  const at::Tensor plan = plan_in.has_value() ? *plan_in : prefill_plan(q, kv_heads, cu_q, cu_k, stream);
+  if (!plan.defined()) return py::none();
+  const int64_t need = g_prefill_workspace(plan.size(0), kv_heads, tables.size(1) * key_cache.size(1));
+  const at::Tensor workspace = need > 0 ? bytes_on(need, q) : at::Tensor();
+  check_status(g_prefill(q.data_ptr(), q.stride(0), key_cache.data_ptr(), value_cache.data_ptr(),
+                         tables.data_ptr<int32_t>(), tables.size(1), cu_q.data_ptr<int32_t>(),
+                         cu_k.data_ptr<int32_t>(), data_or_null(plan), plan.size(0), seqs, kv_heads,
+                         q.size(1), kDim, key_cache.size(1), key_cache.size(0),
+                         static_cast<float>(scale), dtype_code(type), out.data_ptr(), out.stride(0),
+                         need > 0 ? workspace.data_ptr() : nullptr, need,
+                         reinterpret_cast<void*>(stream)),
+               "nanovllm_paged_kv::paged_attention_prefill");
+  return py::cast(out);
+}
+
+// Keys and values back to back, read where they lie: rows of [kv_heads, 128]
+// each in one run, 16-byte aligned.
+py::object varlen(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
+                  const at::Tensor& cu_q, const at::Tensor& cu_k, int64_t max_seqlen_k, double scale,
+                  int64_t stream) {
+  const at::Device device = q.device();
+  const at::ScalarType type = q.scalar_type();
+  if (g_varlen == nullptr || !q.is_cuda() || !half_type(type) || !head_rows(q, type, device) ||
+      !head_rows(k, type, device) || !head_rows(v, type, device) || k.sizes() != v.sizes() ||
+      k.size(0) == 0 || k.size(1) == 0 || !int32_vector(cu_q, device) || !int32_vector(cu_k, device) ||
+      cu_q.size(0) != cu_k.size(0) || cu_q.size(0) < 2 || index_values_checked(cu_k)) {
+    return py::none();
+  }
+  for (const at::Tensor* t : {&k, &v}) {
+    if (t->stride(0) < kDim * t->size(1) || t->stride(0) % 8 != 0 ||
+        reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 != 0) {
+      return py::none();
+    }
+  }
+  const int64_t seqs = cu_q.size(0) - 1, kv_heads = k.size(1);
+  const at::Tensor plan = prefill_plan(q, kv_heads, cu_q, cu_k, stream);
+  if (!plan.defined()) return py::none();
+  const at::Tensor out = at::empty_like(q);
+  const int64_t longest = std::max<int64_t>(max_seqlen_k, 1);
+  const int64_t need = g_prefill_workspace(plan.size(0), kv_heads, longest);
+  const at::Tensor workspace = need > 0 ? bytes_on(need, q) : at::Tensor();
+  check_status(g_varlen(q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(),
+                        v.stride(0), k.size(0), longest, cu_q.data_ptr<int32_t>(),
+                        cu_k.data_ptr<int32_t>(), plan.data_ptr(), plan.size(0), seqs, kv_heads,
+                        q.size(1), kDim, static_cast<float>(scale), dtype_code(type), out.data_ptr(),
+                        out.stride(0), need > 0 ? workspace.data_ptr() : nullptr, need,
+                        reinterpret_cast<void*>(stream)),
+               "nanovllm_paged_kv::varlen_attention_prefill");
+  return py::cast(out);
+}
+
+void bind_attention(uintptr_t decode_capacity, uintptr_t decode_workspace, uintptr_t decode_fn,
+                    uintptr_t prefill_capacity, uintptr_t prefill_plan_fn, uintptr_t prefill_workspace,
+                    uintptr_t prefill_fn, uintptr_t varlen_fn) {
+  g_decode_capacity = reinterpret_cast<PlanCapacityFn>(decode_capacity);
+  g_decode_workspace = reinterpret_cast<WorkspaceFn>(decode_workspace);
+  g_decode = reinterpret_cast<DecodeFn>(decode_fn);
+  g_prefill_capacity = reinterpret_cast<PlanCapacityFn>(prefill_capacity);
+  g_prefill_plan = reinterpret_cast<PrefillPlanFn>(prefill_plan_fn);
+  g_prefill_workspace = reinterpret_cast<WorkspaceFn>(prefill_workspace);
+  g_prefill = reinterpret_cast<PrefillFn>(prefill_fn);
+  g_varlen = reinterpret_cast<VarlenFn>(varlen_fn);
+}
+
 void bind(uintptr_t store_fn, uintptr_t gather_fn, uintptr_t last_error_fn) {
   g_store = reinterpret_cast<StoreFn>(store_fn);
   g_gather = reinterpret_cast<GatherFn>(gather_fn);
@@ -206,6 +393,11 @@ void bind(uintptr_t store_fn, uintptr_t gather_fn, uintptr_t last_error_fn) {
 PYBIND11_MODULE(_nkv_host, m) {
   m.doc() = "Per-call host path of the nanokv hip backend's store and gather";
   m.def("bind", &bind, "set the library entry points (nkv_store, nkv_gather, nkv_last_error)");
+  m.def("bind_attention", &bind_attention, "set the library's attention entry points");
+  m.def("decode", &decode, "planned decode attention; None when the general path has to look at it");
+  m.def("prefill", &prefill, "paged prefill attention; None when the general path has to look at it");
+  m.def("varlen", &varlen, "prefill attention over keys back to back; None when the general path "
+                           "has to look at it");
   m.def("store", &store, "validated store launch on a stream");
   m.def("gather", &gather, "validated gather launch on a stream; returns the new tensor");
   m.def("check_store", &check_store, "the store validator's checks (no launch)");

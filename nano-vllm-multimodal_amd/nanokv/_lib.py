@@ -301,6 +301,11 @@ def load_host():
                 return ctypes.cast(getattr(library, name), ctypes.c_void_p).value
 
             module.bind(address("nkv_store"), address("nkv_gather"), address("nkv_last_error"))
+            module.bind_attention(*(address(name) for name in (
+                "nkv_attention_plan_capacity", "nkv_attention_workspace_bytes",
+                "nkv_paged_attention_decode_total", "nkv_prefill_plan_capacity",
+                "nkv_build_prefill_plan", "nkv_prefill_workspace_bytes",
+                "nkv_paged_attention_prefill_split", "nkv_varlen_attention_prefill")))
             _HOST = module
     return _HOST
 

@@ -21,7 +21,6 @@ import torch
 
 from nanokv.paged_kv.base import index_value_validation_enabled
 from nanokv.paged_kv.hip_backend import HIPPagedKVBackend
-from nanokv.paged_kv.ops import varlen_attention_prefill, varlen_prefill_in_place
 
 _BACKEND = HIPPagedKVBackend()
 _UNSUPPORTED_DEFAULTS = {
@@ -61,13 +60,12 @@ def flash_attn_varlen_func(q, k, v, max_seqlen_q, cu_seqlens_q, max_seqlen_k, cu
         # Keys back to back are read where they lie, views of the fused
         # projection included: compacting them, building a table for them
         # and sorting the plan were five launches beside the attention,
-        # 23 us of a 1,511-token prompt's 62.  (The host-side value checks
-        # of index validation belong to the paged path.)
-        if (not index_value_validation_enabled(cu_seqlens_k)
-                and varlen_prefill_in_place(q, k, v, cu_seqlens_q, cu_seqlens_k)):
-            _BACKEND._load()
-            return varlen_attention_prefill(q, k, v, cu_seqlens_q, cu_seqlens_k,
-                                            max(1, int(max_seqlen_k)), scale)
+        # 23 us of a 1,511-token prompt's 62.  (None: not as the kernels take
+        # them, or index values are to be checked.)
+        out = _BACKEND.varlen_attention_prefill(q, k, v, cu_seqlens_q, cu_seqlens_k,
+                                                int(max_seqlen_k), scale)
+        if out is not None:
+            return out
         # Otherwise: a cache of one-row blocks whose table for request i
         # counts up from cu_seqlens_k[i] (entries past its length are never
         # read).

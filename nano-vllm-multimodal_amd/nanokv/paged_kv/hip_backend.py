@@ -323,6 +323,19 @@ class HIPPagedKVBackend:
         SDPAAttention's decode branch (attention.py:284-300), without the
         gather.  q [B, Hq, 128] bf16 or fp16 (the caches' type) -> [B, Hq, 128]
         in that type."""
+        # A planned call with everything as the kernels take it runs in the
+        # host binding (csrc/nkv_host.cpp); None: the checks below decide.
+        if plan is not None:
+            if not _READY:
+                self._load()
+            built_for = getattr(plan, "lengths", None)
+            if built_for is None or built_for == (total_tokens, block_tables.shape[0], key_cache.shape[2]):
+                index = q.get_device()
+                done = _HOST.decode(q, key_cache, value_cache, block_tables, cu_seqlens_k, plan[0],
+                                    plan[1], int(total_tokens), float(softmax_scale), out,
+                                    ops.stream_of(index) if index >= 0 else 0)
+                if done is not None:
+                    return done if out is None else out
         validate_varlen_inputs(key_cache, value_cache, block_tables, cu_seqlens_k, total_tokens)
         if q.ndim != 3 or q.shape[0] != block_tables.shape[0]:
             raise ValueError("q must be [num_seqs, num_q_heads, head_dim] with one row per sequence")
@@ -352,6 +365,17 @@ class HIPPagedKVBackend:
             int(total_tokens),
         )
         return out
+
+    def varlen_attention_prefill(self, q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_k: int,
+                                 softmax_scale: float) -> torch.Tensor | None:
+        """Causal attention over keys and values that lie back to back
+        [total_k, kv_heads, 128], read in place (views of the fused
+        projection included); None where the paged path has to serve."""
+        if not _READY:
+            self._load()
+        index = q.get_device()
+        return _HOST.varlen(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_k, softmax_scale,
+                            ops.stream_of(index) if index >= 0 else 0)
 
     def build_prefill_plan(self, q: torch.Tensor, key_cache: torch.Tensor,
                            cu_seqlens_q: torch.Tensor, cu_seqlens_k: torch.Tensor) -> torch.Tensor:
@@ -387,6 +411,13 @@ class HIPPagedKVBackend:
         ``total_context_tokens`` (= cu_seqlens_k[-1]) is only read by the
         host-side value checks of index validation (read from the device
         when not given)."""
+        if not _READY:
+            self._load()
+        index = q.get_device()
+        done = _HOST.prefill(q, key_cache, value_cache, block_tables, cu_seqlens_q, cu_seqlens_k, plan,
+                             float(softmax_scale), out, ops.stream_of(index) if index >= 0 else 0)
+        if done is not None:
+            return done if out is None else out
         from nanokv.paged_kv.base import index_value_validation_enabled
 
         total = total_context_tokens

@@ -545,46 +545,6 @@ def _paged_attention_prefill_impl(q, key_cache, value_cache, block_tables, cu_se
     _lib.check(status, "nanovllm_paged_kv::paged_attention_prefill")
 
 
-def varlen_prefill_in_place(q, k, v, cu_seqlens_q, cu_seqlens_k) -> bool:
-    """Whether :func:`varlen_attention_prefill` takes these tensors as they
-    are: rows of [kv_heads, 128] each in one run, 16-byte aligned, int32
-    offsets, one GPU.  The paged path serves (or refuses) everything else."""
-    return bool(
-        q.is_cuda and q.ndim == 3 and k.ndim == 3 and k.shape == v.shape
-        and q.dtype in (torch.bfloat16, torch.float16) and k.dtype == q.dtype and v.dtype == q.dtype
-        and q.shape[2] == 128 and k.shape[2] == 128 and k.shape[1] > 0 and k.shape[0] > 0
-        and q.stride(2) == 1 and q.stride(1) == 128
-        and all(t.stride(2) == 1 and t.stride(1) == 128 and t.stride(0) >= 128 * t.shape[1]
-                and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0 for t in (k, v))
-        and all(cu.dtype == torch.int32 and cu.ndim == 1 and cu.is_contiguous() and cu.numel() > 1
-                for cu in (cu_seqlens_q, cu_seqlens_k))
-        and cu_seqlens_q.numel() == cu_seqlens_k.numel()
-        and len({t.device for t in (q, k, v, cu_seqlens_q, cu_seqlens_k)}) == 1
-    )
-
-
-def varlen_attention_prefill(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_k: int,
-                             scale: float) -> torch.Tensor:
-    """Prefill attention over keys and values read where they lie, for
-    tensors :func:`varlen_prefill_in_place` accepts."""
-    device = q.device
-    num_seqs, num_kv_heads = cu_seqlens_q.numel() - 1, k.shape[1]
-    plan = _build_prefill_plan_impl(cu_seqlens_q, cu_seqlens_k, q.shape[0], q.shape[1] // num_kv_heads)
-    out = torch.empty_like(q)
-    library = _lib.load_library()
-    nbytes = int(library.nkv_prefill_workspace_bytes(plan.shape[0], num_kv_heads, max_seqlen_k))
-    workspace = torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None
-    status = library.nkv_varlen_attention_prefill(
-        q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(), v.stride(0), k.shape[0],
-        max_seqlen_k, cu_seqlens_q.data_ptr(), cu_seqlens_k.data_ptr(),
-        plan.data_ptr() if plan.shape[0] else None, plan.shape[0], num_seqs, num_kv_heads,
-        q.shape[1], 128, scale, DTYPE_CODES[q.dtype], out.data_ptr(), out.stride(0),
-        workspace.data_ptr() if nbytes else None, nbytes, _stream(device),
-    )
-    _lib.check(status, "nanovllm_paged_kv::varlen_attention_prefill")
-    return out
-
-
 def register_ops() -> None:
     """Define the schemas (unless another library already did) and register
     the HIP implementations on the CUDA key.  Idempotent."""

@@ -581,3 +581,35 @@ def test_plan_from_lengths_equals_plan_from_offsets(backend, gpu_device, hkv, le
     assert torch.equal(one[1], other[1])
     used = int(one[1][-1]) if hkv >= 8 else 1 + 1024  # entries, or the header and the workers' records
     assert torch.equal(one[0][:used], other[0][:used])
+
+
+@pytest.mark.parametrize("hkv,g,pad", [(8, 2, 0), (4, 7, 3), (2, 16, 1)])
+def test_host_binding_equals_the_general_path(backend, gpu_device, monkeypatch, hkv, g, pad):
+    """Decode and prefill through the host binding and through the Python
+    checks: the same bits, new and given outputs, a strided q."""
+    from nanokv.paged_kv import hip_backend
+
+    lens = [300, 1, 513, 40]
+    dev, host, total = build_case(gpu_device, hkv, g, 16, lens, seed=hkv, q_pad_heads=pad)
+    plan = backend.build_attention_plan(dev["kc"], dev["cu"], total)
+    cu_q = torch.arange(len(lens) + 1, dtype=torch.int32, device=gpu_device)  # one query each
+
+    def calls():
+        outs = []
+        for make in (lambda: None, lambda: torch.zeros_like(dev["q"].contiguous())):
+            outs.append(backend.paged_attention_decode(dev["q"], dev["kc"], dev["vc"], dev["tables"],
+                                                       dev["cu"], total, 0.1, plan=plan, out=make()))
+            if g <= 8:
+                outs.append(backend.paged_attention_prefill(dev["q"], dev["kc"], dev["vc"], dev["tables"],
+                                                            cu_q, dev["cu"], 0.1, out=make()))
+        return outs
+
+    native = calls()
+    taken = []
+    for name in ("decode", "prefill"):
+        monkeypatch.setattr(hip_backend._HOST, name, lambda *a, name=name: taken.append(name))
+    general = calls()
+    assert taken
+    for a, b in zip(native, general):
+        assert torch.equal(a, b)
+    check_close(native[0], reference(host, 0.1), "native decode")

@@ -455,8 +455,9 @@ def test_flash_varlen_in_place_equals_the_paged_path(gpu_device, monkeypatch, hk
     for view, rows_of in zip(views, (k, v)):
         view.copy_(rows_of.view(total, width))
     k, v = (view.unflatten(1, (hkv, 128)) for view in views)
-    assert flash.varlen_prefill_in_place(dev["q"], k, v, dev["cu_q"], dev["cu_k"]) == (layout != "odd")
     max_k = max(k_lens) - (21 if layout == "short" else 0)
+    in_place = flash._BACKEND.varlen_attention_prefill(dev["q"], k, v, dev["cu_q"], dev["cu_k"], max_k, 0.1)
+    assert (in_place is None) == (layout == "odd")
 
     def call():
         return flash.flash_attn_varlen_func(dev["q"], k, v, max(q_lens), dev["cu_q"], max_k, dev["cu_k"],
@@ -465,7 +466,7 @@ def test_flash_varlen_in_place_equals_the_paged_path(gpu_device, monkeypatch, hk
     out = call()
     if layout != "short":
         check_close(out, *reference(host, 0.1), f"{layout} hkv={hkv} g={g}")
-    monkeypatch.setattr(flash, "varlen_prefill_in_place", lambda *a: False)
+    monkeypatch.setattr(flash._BACKEND, "varlen_attention_prefill", lambda *a: None, raising=False)
     assert torch.equal(out, call())
 
 

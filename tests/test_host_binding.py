@@ -125,3 +125,23 @@ def test_graph_buffers_collect_dead_cycles_before_a_capture():
     del holder
     DecodeGraphBuffers.allocate("cpu", 2, 3)
     assert dead() is None
+
+
+def test_attention_calls_the_binding_leaves_to_the_general_path():
+    """Host tensors, and calls any check of the general path looks into, are
+    not taken by the binding's attention entries: they return None, and the
+    backend's own checks answer."""
+    import torch
+
+    from nanokv import _lib
+
+    host = _lib.load_host()
+    q = torch.zeros((2, 4, 128), dtype=torch.bfloat16)
+    cache = torch.zeros((3, 16, 2, 128), dtype=torch.bfloat16)
+    tables = torch.zeros((2, 1), dtype=torch.int32)
+    cu = torch.tensor([0, 1, 2], dtype=torch.int32)
+    plan = torch.zeros((1030, 4), dtype=torch.int32)
+    assert host.decode(q, cache, cache, tables, cu, plan, cu, 2, 0.1, None, 0) is None
+    assert host.prefill(q, cache, cache, tables, cu, cu, None, 0.1, None, 0) is None
+    rows = torch.zeros((2, 2, 128), dtype=torch.bfloat16)
+    assert host.varlen(q, rows, rows, cu, cu, 1, 0.1, 0) is None
