@@ -383,7 +383,8 @@ __device__ __forceinline__ Piece find_piece(const int4* __restrict__ plan, int32
     count[i] = 0;
     if (i < per && lane * per + i < capacity) {
       const int4 e = plan[lane * per + i];
-      if (e.z > 0 && e.w > 0) count[i] = min(e.w, kSplitTileClamp);
+      // A plan written without the key tiles gets one piece per query tile.
+      if (e.z > 0) count[i] = min(max(e.w, 1), kSplitTileClamp);
     }
   }
 #pragma unroll
@@ -457,7 +458,7 @@ __global__ __launch_bounds__(kMergeWaves* kWave) void prefill_merge_kernel(
   const int32_t seq = entry.x;
   const int32_t tok0 = entry.y;
   const int32_t ntok = entry.z;
-  if (ntok <= 0 || entry.w <= 0 || ntok > kPfRows / group || seq < 0 || seq >= num_seqs || tok0 < 0) return;
+  if (ntok <= 0 || ntok > kPfRows / group || seq < 0 || seq >= num_seqs || tok0 < 0) return;
   const int2 parts = tile_parts[e];  // {first partial, pieces}
   const int32_t q_begin = cu_seqlens_q[seq];
   const int32_t lq = cu_seqlens_q[seq + 1] - q_begin;

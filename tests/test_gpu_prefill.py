@@ -149,6 +149,10 @@ def test_short_launches_cut_their_keys(backend, gpu_device, hkv, g, bs, q_lens, 
         ops.DTYPE_CODES[dtype], whole.data_ptr(), whole.stride(0),
         ops.current_stream_handle(gpu_device)), "prefill without a workspace")
     check_close(out, whole.float().cpu().numpy(), ref_abs, "dropped blocks")
+    plan[:, 3] = 0  # a plan that does not say what its tiles see: nothing is cut
+    uncut = torch.full_like(out, float("nan"))
+    run(backend, dev, scale, plan=plan, out=uncut)
+    assert torch.equal(uncut, whole)
 
 
 def check_plan(plan, q_lens, k_lens, tile, longest_first):
