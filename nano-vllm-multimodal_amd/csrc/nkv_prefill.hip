@@ -317,8 +317,8 @@ __device__ __forceinline__ TileId tile_of(uint32_t id, int32_t num_kv_heads, int
 // and took 262 us, 195 key tiles in a row on a quarter of the CUs.  Such a
 // launch cuts each tile's keys into pieces of at most C key tiles, one
 // workgroup each, whose fp32 partials (max, weight sum, output sums) a merge
-// kernel adds up: that case went to 56-62 us, one 40-token chunk over 14k
-// cached rows from 311 to 38 us.
+// kernel adds up: that case went to 57 us, one 40-token chunk over 14k
+// cached rows from 311 to 33 us.
 // One kv head can have slots = 512 / Hkv workgroups resident at once (two
 // per CU).  With T key tiles in the whole plan, C = T / (slots - tiles)
 // makes at most T / C + tiles <= slots pieces, which start together; more
@@ -433,12 +433,18 @@ __device__ __forceinline__ Piece find_piece(const int4* __restrict__ plan, int32
 }
 
 // Adds the partials of the tiles that were cut.  A wavefront merges 16 rows
-// x 64 dims of one (tile, kv head); a lane holds the same row and dims as in
+// x 32 dims of one (tile, kv head); a lane holds the same row and dims as in
 // the attention kernel, so the row's weights need no exchange and every
-// access is 1 KiB.  Four pieces are in flight at once.
+// access is 1 KiB.  Four pieces are in flight at once.  It waits for memory,
+// so more and smaller wavefronts help: with 64 dims each, one 40-token chunk
+// over 14k cached rows (56 pieces a tile) took 36.7 us instead of 32.7, the
+// other launches up to 1% more; 16 dims and eight pieces in flight were 2%
+// slower on those.  Blocks of padding rows are neither written nor read.
 constexpr int kMergeBatch = 4;
 constexpr int kMergeWaves = 4;
-constexpr int kMergeUnits = kPfRows / 16 * 2;  // wavefronts per (tile, kv head)
+constexpr int kMergeParts = 4;  // wavefronts per 16 rows
+constexpr int kMergeDims = 8 / kMergeParts;               // 16-dim blocks per wavefront
+constexpr int kMergeUnits = kPfRows / 16 * kMergeParts;  // wavefronts per (tile, kv head)
 static_assert(kMergeUnits % kMergeWaves == 0, "whole workgroups per tile");
 
 template <bool kHalf>
@@ -468,16 +474,17 @@ __global__ __launch_bounds__(kMergeWaves* kWave) void prefill_merge_kernel(
   const int lane = threadIdx.x & (kWave - 1);
   const int unit = static_cast<int>(blockIdx.x) % kBlocksPerTile * kMergeWaves +
                    __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int block = unit >> 1;       // 16-row block
-  const int db0 = (unit & 1) * 4;    // first 16-dim block
+  const int block = unit / kMergeParts;                // 16-row block
+  const int db0 = unit % kMergeParts * kMergeDims;     // first 16-dim block
+  if (block * 16 >= ntok * group) return;              // padding rows only
   const int m = block * 16 + (lane & 15);
   float run_max = -INFINITY, run_sum = 0.f;
-  f32x4 acc[4];
+  f32x4 acc[kMergeDims];
 #pragma unroll
-  for (int d = 0; d < 4; ++d) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int d = 0; d < kMergeDims; ++d) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int32_t p = 0; p < parts.y; p += kMergeBatch) {
     f32x2 ml[kMergeBatch];
-    f32x4 v[kMergeBatch][4];
+    f32x4 v[kMergeBatch][kMergeDims];
 #pragma unroll
     for (int i = 0; i < kMergeBatch; ++i) {
       const int64_t slot =
@@ -486,7 +493,7 @@ __global__ __launch_bounds__(kMergeWaves* kWave) void prefill_merge_kernel(
       const f32x4* src = reinterpret_cast<const f32x4*>(part_acc + slot * kPartSums) +
                          (block * 8 + db0) * kWave + lane;
 #pragma unroll
-      for (int d = 0; d < 4; ++d) v[i][d] = src[d * kWave];
+      for (int d = 0; d < kMergeDims; ++d) v[i][d] = src[d * kWave];
     }
     float top = run_max;
 #pragma unroll
@@ -497,7 +504,7 @@ __global__ __launch_bounds__(kMergeWaves* kWave) void prefill_merge_kernel(
     const float keep = run_max == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(run_max - top);
     run_sum *= keep;
 #pragma unroll
-    for (int d = 0; d < 4; ++d) acc[d] *= keep;
+    for (int d = 0; d < kMergeDims; ++d) acc[d] *= keep;
 #pragma unroll
     for (int i = 0; i < kMergeBatch; ++i) {
       // A piece without visible keys has max -inf and sum 0 (and, with no
@@ -507,7 +514,7 @@ __global__ __launch_bounds__(kMergeWaves* kWave) void prefill_merge_kernel(
       const float f = ml[i].x == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(ml[i].x - top);
       run_sum = __builtin_fmaf(ml[i].y, f, run_sum);
 #pragma unroll
-      for (int d = 0; d < 4; ++d) {
+      for (int d = 0; d < kMergeDims; ++d) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[d][j] = __builtin_fmaf(v[i][d][j], f, acc[d][j]);
       }
@@ -520,7 +527,7 @@ __global__ __launch_bounds__(kMergeWaves* kWave) void prefill_merge_kernel(
   uint16_t* orow = out + static_cast<int64_t>(q_begin + tok0 + t) * out_token_stride +
                    (kh * group + m % group) * kPfDim + 16 * db0 + 4 * (lane >> 4);
 #pragma unroll
-  for (int d = 0; d < 4; ++d) {
+  for (int d = 0; d < kMergeDims; ++d) {
     const X4 w = {static_cast<T>(acc[d].x * inv), static_cast<T>(acc[d].y * inv),
                   static_cast<T>(acc[d].z * inv), static_cast<T>(acc[d].w * inv)};
     *reinterpret_cast<X4*>(orow + 16 * d) = w;
@@ -835,8 +842,9 @@ __global__ __launch_bounds__(kPfThreads, kPfBlocksPerCU) void attn_prefill_kerne
     const float total = row4_sum(g4 == 0 ? acc[8][mb][0] : 0.f);
     const int m = wave * 32 + mb * 16 + c16;
     const int t = m / G;
-    if (kSplit && part.pieces > 1) {  // this piece's partial, padding rows included (the merge skips them)
+    if (kSplit && part.pieces > 1) {  // this piece's partial
       const int block = wave * 2 + mb;
+      if (block * 16 >= ntok * G) continue;  // padding rows only: not merged either
       if (g4 == 0) part_ml[part_slot * kPfRows + block * 16 + c16] = f32x2{row_max[mb], total};
       f32x4* dst = reinterpret_cast<f32x4*>(part_acc + part_slot * kPartSums) + block * 8 * kWave + lane;
 #pragma unroll
