@@ -174,7 +174,7 @@ __device__ __forceinline__ void wait_lgkmcnt0() {
 // lds_dst + 4 l (global_load_lds_dword, LDS base in M0), counted like the
 // 16-byte copies of nkv_mfma.h.
 __device__ __forceinline__ void lds_copy4(const int32_t* src, uint32_t lds_dst) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off"
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
                :
                : "v"(src), "s"(lds_dst)
                : "m0", "memory");

@@ -88,6 +88,10 @@ __device__ __forceinline__ float row4_sum(float x) {
 // preserved; in the kernels built from this file every M0 access is the
 // s_mov_b32 or s_add_u32 of these copies (no compiler value lives in M0
 // across them).
+// A scalar write of M0 needs one wait state before a load into LDS reads it
+// (the s_nop; the compiler puts one there itself, but not inside asm): the
+// next instruction may otherwise still see the old M0 and write the copy
+// over the previous one's rows.
 // LDS byte address of a __shared__ array (a constant once inlined).
 __device__ __forceinline__ uint32_t lds_address(const u32x4* array) {
   typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
@@ -98,12 +102,12 @@ __device__ __forceinline__ uint32_t lds_address(const u32x4* array) {
 template <bool kStream = false>
 __device__ __forceinline__ void lds_copy16(const uint8_t* src, uint32_t lds_dst) {
   if constexpr (kStream) {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off nt"
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off nt"
                  :
                  : "v"(src), "s"(lds_dst)
                  : "m0", "memory");
   } else {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off"
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
                  :
                  : "v"(src), "s"(lds_dst)
                  : "m0", "memory");
@@ -113,12 +117,12 @@ __device__ __forceinline__ void lds_copy16(const uint8_t* src, uint32_t lds_dst)
 template <bool kStream = false>
 __device__ __forceinline__ void lds_copy16(const uint8_t* base, uint32_t offset, uint32_t lds_dst) {
   if constexpr (kStream) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1 nt"
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt"
                  :
                  : "v"(offset), "s"(base), "s"(lds_dst)
                  : "m0", "memory");
   } else {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1"
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                  :
                  : "v"(offset), "s"(base), "s"(lds_dst)
                  : "m0", "memory");
@@ -130,14 +134,14 @@ __device__ __forceinline__ void lds_copy16(const uint8_t* base, uint32_t offset,
 // prefill kernel's scalars into lane spills).
 template <int kDst>
 __device__ __forceinline__ void lds_copy16_at(const uint8_t* src, uint32_t lds_dst) {
-  asm volatile("s_add_u32 m0, %1, %2\n\tglobal_load_lds_dwordx4 %0, off"
+  asm volatile("s_add_u32 m0, %1, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
                :
                : "v"(src), "s"(lds_dst), "n"(kDst)
                : "m0", "scc", "memory");
 }
 template <int kDst>
 __device__ __forceinline__ void lds_copy16_at(const uint8_t* base, uint32_t offset, uint32_t lds_dst) {
-  asm volatile("s_add_u32 m0, %2, %3\n\tglobal_load_lds_dwordx4 %0, %1"
+  asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                :
                : "v"(offset), "s"(base), "s"(lds_dst), "n"(kDst)
                : "m0", "scc", "memory");
