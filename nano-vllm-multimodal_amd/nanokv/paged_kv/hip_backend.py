@@ -413,11 +413,15 @@ class HIPPagedKVBackend:
         when not given)."""
         if not _READY:
             self._load()
-        index = q.get_device()
-        done = _HOST.prefill(q, key_cache, value_cache, block_tables, cu_seqlens_q, cu_seqlens_k, plan,
-                             float(softmax_scale), out, ops.stream_of(index) if index >= 0 else 0)
-        if done is not None:
-            return done if out is None else out
+        # The host binding never reads the total: a negative one is the
+        # general path's to refuse.
+        if total_context_tokens is None or int(total_context_tokens) >= 0:
+            index = q.get_device()
+            done = _HOST.prefill(q, key_cache, value_cache, block_tables, cu_seqlens_q, cu_seqlens_k,
+                                 plan, float(softmax_scale), out,
+                                 ops.stream_of(index) if index >= 0 else 0)
+            if done is not None:
+                return done if out is None else out
         from nanokv.paged_kv.base import index_value_validation_enabled
 
         total = total_context_tokens

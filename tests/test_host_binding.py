@@ -145,3 +145,26 @@ def test_attention_calls_the_binding_leaves_to_the_general_path():
     assert host.prefill(q, cache, cache, tables, cu, cu, None, 0.1, None, 0) is None
     rows = torch.zeros((2, 2, 128), dtype=torch.bfloat16)
     assert host.varlen(q, rows, rows, cu, cu, 1, 0.1, 0) is None
+
+
+@pytest.mark.parametrize("total,error", [(-1, ValueError), ("many", ValueError), ([3], TypeError)])
+def test_prefill_refuses_a_bad_context_total_before_the_binding(host, monkeypatch, total, error):
+    """The binding does not read total_context_tokens; what the general path
+    refuses there never reaches it."""
+    from nanokv.paged_kv import hip_backend
+
+    backend = hip_backend.HIPPagedKVBackend()
+    backend._load()
+
+    class Taken:
+        prefill = staticmethod(lambda *args: "taken")
+
+    monkeypatch.setattr(hip_backend, "_HOST", Taken)
+    q = torch.zeros((3, 4, 128), dtype=torch.bfloat16)
+    cache = torch.zeros((3, 16, 2, 128), dtype=torch.bfloat16)
+    tables = torch.zeros((2, 1), dtype=torch.int32)
+    cu = torch.tensor([0, 1, 3], dtype=torch.int32)
+    args = (q, cache, cache, tables, cu, cu, 0.1)
+    assert backend.paged_attention_prefill(*args, total_context_tokens=3) == "taken"
+    with pytest.raises(error):
+        backend.paged_attention_prefill(*args, total_context_tokens=total)
