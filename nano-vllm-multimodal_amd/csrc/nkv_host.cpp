@@ -252,21 +252,26 @@ at::Tensor bytes_on(int64_t bytes, const at::Tensor& like) {
 }
 void* data_or_null(const at::Tensor& t) { return t.size(0) > 0 ? t.data_ptr() : nullptr; }
 
+// The offsets are only checked (the plan holds what the kernels need);
+// callers that built the plan from the lengths have none.
 py::object decode(const at::Tensor& q, const at::Tensor& key_cache, const at::Tensor& value_cache,
-                  const at::Tensor& tables, const at::Tensor& cu_seqlens_k, const at::Tensor& plan,
-                  const at::Tensor& first_part, int64_t total_tokens, double scale,
-                  const c10::optional<at::Tensor>& out_in, int64_t stream) {
+                  const at::Tensor& tables, const c10::optional<at::Tensor>& cu_seqlens_k,
+                  const at::Tensor& plan, const at::Tensor& first_part, int64_t total_tokens,
+                  double scale, const c10::optional<at::Tensor>& out_in, int64_t stream) {
   const at::Device device = q.device();
   const at::ScalarType type = q.scalar_type();
   if (g_decode == nullptr || !q.is_cuda() || !half_type(type) || !head_rows(q, type, device) ||
       !caches(key_cache, value_cache, type, device) || !int32_matrix(tables, device) ||
-      !int32_vector(cu_seqlens_k, device) || !int32_matrix(plan, device) ||
-      !int32_vector(first_part, device) || total_tokens < 0 || index_values_checked(cu_seqlens_k)) {
+      !int32_matrix(plan, device) || !int32_vector(first_part, device) || total_tokens < 0 ||
+      index_values_checked(tables)) {
     return py::none();
   }
   const int64_t seqs = q.size(0);
-  if (seqs == 0 || tables.size(0) != seqs || cu_seqlens_k.size(0) != seqs + 1 ||
-      first_part.size(0) != seqs + 1 || plan.size(1) != 4 ||
+  if (cu_seqlens_k.has_value() &&
+      (!int32_vector(*cu_seqlens_k, device) || cu_seqlens_k->size(0) != seqs + 1)) {
+    return py::none();
+  }
+  if (seqs == 0 || tables.size(0) != seqs || first_part.size(0) != seqs + 1 || plan.size(1) != 4 ||
       plan.size(0) < g_decode_capacity(total_tokens, seqs, key_cache.size(1))) {
     return py::none();
   }

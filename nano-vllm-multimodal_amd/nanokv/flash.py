@@ -145,13 +145,12 @@ def flash_attn_with_kvcache(q, k_cache, v_cache, cache_seqlens=None, block_table
         lengths = cache_seqlens.to(device=q.device, dtype=torch.int32)
         if (capturing and lengths.shape == (batch,) and lengths.is_contiguous()
                 and not index_value_validation_enabled(lengths)):
-            # One planning launch per layer of the graph; the plan's
-            # first_part stands in for the offsets, which nothing reads
-            # once there is a plan.
+            # One planning launch per layer of the graph, and no offsets.
             total = batch * block_table.shape[1] * k_cache.shape[1]
-            plan = _BACKEND.build_attention_plan_from_lengths(k_cache, lengths, total)
-            return _BACKEND.paged_attention_decode(q[:, 0], k_cache, v_cache, block_table, plan[1],
-                                                   total, scale, plan=plan).unsqueeze(1)
+            out = _BACKEND.paged_attention_decode_lengths(q[:, 0], k_cache, v_cache, block_table,
+                                                          lengths, total, scale)
+            if out is not None:
+                return out.unsqueeze(1)
         cu_seqlens_k = torch.zeros(batch + 1, dtype=torch.int32, device=q.device)
         torch.cumsum(lengths, 0, out=cu_seqlens_k[1:])
         if capturing and not index_value_validation_enabled(lengths):

@@ -366,6 +366,17 @@ class HIPPagedKVBackend:
         )
         return out
 
+    def paged_attention_decode_lengths(self, q, key_cache, value_cache, block_tables, context_lens,
+                                       total_tokens: int, softmax_scale: float) -> torch.Tensor | None:
+        """:meth:`paged_attention_decode` from the context lengths themselves
+        (contiguous 1-D int32), planned and run without their offsets; None
+        where the general path, which checks the offsets, has to look."""
+        plan = self.build_attention_plan_from_lengths(key_cache, context_lens, total_tokens)
+        index = q.get_device()
+        return _HOST.decode(q, key_cache, value_cache, block_tables, None, plan[0], plan[1],
+                            total_tokens, softmax_scale, None,
+                            ops.stream_of(index) if index >= 0 else 0)
+
     def varlen_attention_prefill(self, q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_k: int,
                                  softmax_scale: float) -> torch.Tensor | None:
         """Causal attention over keys and values that lie back to back

@@ -6,8 +6,10 @@ from __future__ import annotations
 
 import gc
 
+import pytest
 import torch
 
+from nanokv import flash
 from nanokv.flash import _StepPlan
 
 
@@ -66,3 +68,36 @@ def test_a_different_block_size_or_shape_is_a_miss():
     lengths = torch.tensor([3, 5, 7], dtype=torch.int32)
     plans.store(lengths, key_of(lengths, 16), 100, "cu", 15, "plan")
     assert plans.lookup(lengths, key_of(lengths, 32), 200) is None
+
+
+@pytest.mark.parametrize("binding_serves", [True, False])
+def test_captured_decode_never_passes_a_plan_as_offsets(monkeypatch, binding_serves):
+    """Under capture the plan comes from the lengths, and there are no
+    offsets.  A call that the host binding leaves to the general path gets
+    real ones: that path checks them."""
+    seen = []
+
+    class Backend:
+        def build_attention_plan_from_lengths(self, cache, lengths, total):
+            return torch.full((4, 4), 7, dtype=torch.int32), torch.full((4,), 9, dtype=torch.int32)
+
+        def paged_attention_decode_lengths(self, q, k, v, tables, lengths, total, scale):
+            seen.append(("lengths", lengths.tolist(), total))
+            return q if binding_serves else None
+
+        def paged_attention_decode(self, q, k, v, tables, cu_seqlens_k, total, scale, plan=None):
+            seen.append(("offsets", cu_seqlens_k.tolist(), total))
+            return q
+
+    monkeypatch.setattr(flash, "_BACKEND", Backend())
+    monkeypatch.setattr(flash, "index_value_validation_enabled", lambda tensor: False)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    q, cache = torch.zeros(3, 1, 4, 128), torch.zeros(5, 16, 2, 128)
+    lengths = torch.tensor([3, 0, 20], dtype=torch.int32)
+    out = flash.flash_attn_with_kvcache(q, cache, cache, cache_seqlens=lengths,
+                                        block_table=torch.zeros(3, 2, dtype=torch.int32), causal=True)
+    assert out.shape == q.shape
+    expected = [("lengths", [3, 0, 20], 96)]
+    if not binding_serves:
+        expected.append(("offsets", [0, 3, 3, 23], 96))
+    assert seen == expected
