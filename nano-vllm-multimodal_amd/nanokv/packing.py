@@ -18,6 +18,8 @@ from __future__ import annotations
 
 import ctypes
 import gc
+import threading
+from contextlib import contextmanager
 from dataclasses import dataclass
 from typing import Iterable, Sequence
 
@@ -153,11 +155,11 @@ class DecodeGraphBuffers:
             raise ValueError("max_num_seqs and max_blocks must be positive")
         if max_num_seqs > _lib.NKV_MAX_PACK_SEQS:
             raise ValueError(f"at most {_lib.NKV_MAX_PACK_SEQS} sequences per decode graph")
-        # A capture follows.  PyTorch-ROCm's CUDAGraph destructor synchronises
-        # the device, which is an error while a stream captures and ends the
-        # process: a graph that only a reference cycle still holds is freed
-        # now, not by a garbage collection in the middle of the capture.
-        gc.collect()
+        # A capture usually follows.  Collecting the young objects (not the
+        # whole heap, 20 ms) frees the graph of a state just dropped, and no
+        # automatic collection is due for the next several hundred objects.
+        # Only capture_graph guarantees that none runs inside the capture.
+        gc.collect(1)
         device = torch.device(device)
         zeros = lambda *shape: torch.zeros(shape, dtype=torch.int32, device=device)  # noqa: E731
         return cls(zeros(max_num_seqs), zeros(max_num_seqs), zeros(max_num_seqs, max_blocks),
@@ -174,6 +176,37 @@ class DecodeGraphBuffers:
     @property
     def device(self) -> torch.device:
         return self.slot_mapping.device
+
+
+_CAPTURES = 0              # captures under way, and whether the first one
+_COLLECTOR_WAS_ON = False  # found the garbage collector on
+_CAPTURES_LOCK = threading.Lock()
+
+
+@contextmanager
+def capture_graph(graph, **options):
+    """``torch.cuda.graph(graph, **options)`` that no garbage collection can
+    interrupt.  PyTorch-ROCm's CUDAGraph destructor synchronises the device,
+    which is an error while a stream captures and ends the process: a graph
+    that only a reference cycle still holds must not be collected by chance
+    in the middle of another's capture.  What is dead is collected first
+    (the whole heap, some 20 ms), and the automatic collector stays off
+    until the last capture under way has ended."""
+    global _CAPTURES, _COLLECTOR_WAS_ON
+    gc.collect()
+    with _CAPTURES_LOCK:
+        if _CAPTURES == 0:
+            _COLLECTOR_WAS_ON = gc.isenabled()
+        _CAPTURES += 1
+        gc.disable()
+    try:
+        with torch.cuda.graph(graph, **options):
+            yield graph
+    finally:
+        with _CAPTURES_LOCK:
+            _CAPTURES -= 1
+            if _CAPTURES == 0 and _COLLECTOR_WAS_ON:
+                gc.enable()
 
 
 class DevicePacker:

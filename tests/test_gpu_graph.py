@@ -205,3 +205,55 @@ def test_captured_flash_decode_replays_match_oracle(gpu_device, kv_heads, q_head
             assert not got[num_seqs:].any(), f"replay {replay} layer {layer}: padding rows not zero"
         np.testing.assert_array_equal(cache.cpu().view(torch.int16).numpy(), host,
                                       err_msg=f"replay {replay}")
+
+
+def test_captures_with_a_dead_graph_around(gpu_device):
+    """Buffers allocated once serve several captures, and a state holding a
+    graph dies in a reference cycle between two of them: capture_graph frees
+    it before it captures, and both graphs replay what the eager calls give."""
+    import gc
+    import weakref
+
+    from nanokv.flash import flash_attn_with_kvcache
+    from nanokv.packing import DecodeGraphBuffers, DevicePacker, SequenceBatch, capture_graph
+
+    rng = np.random.default_rng(5)
+    cache = torch.randn((2, 64, BS, 8, 128), device=gpu_device).to(torch.bfloat16)
+    q = torch.randn((8, 1, 16, 128), device=gpu_device).to(torch.bfloat16)
+    buffers = DecodeGraphBuffers.allocate(gpu_device, max_num_seqs=8, max_blocks=6)
+    packer = DevicePacker(gpu_device, BS)
+
+    def attend(bucket):
+        return flash_attn_with_kvcache(q[:bucket], cache[0], cache[1],
+                                       cache_seqlens=buffers.context_lens[:bucket],
+                                       block_table=buffers.block_tables[:bucket],
+                                       softmax_scale=0.1, causal=True)
+
+    class State:
+        pass
+
+    def captured(bucket):
+        state = State()
+        attend(bucket)
+        torch.cuda.synchronize()
+        state.graph = torch.cuda.CUDAGraph()
+        with capture_graph(state.graph):
+            state.out = attend(bucket)
+        torch.cuda.synchronize()
+        return state
+
+    n, tables = random_batch(rng, 4, 6 * BS, 64)
+    packer.pack_decode_into(SequenceBatch.from_block_lists(n, tables), buffers)
+    first = captured(8)
+    first.self = first  # only a collection frees it
+    dead = weakref.ref(first)
+    del first
+    small, large = captured(4), captured(8)
+    assert dead() is None and gc.isenabled()
+    for num_seqs in (4, 1, 3):
+        n, tables = random_batch(rng, num_seqs, 6 * BS, 64)
+        packer.pack_decode_into(SequenceBatch.from_block_lists(n, tables), buffers)
+        for state, bucket in ((small, 4), (large, 8)):
+            state.graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(state.out, attend(bucket)), (num_seqs, bucket)

@@ -127,6 +127,75 @@ def test_graph_buffers_collect_dead_cycles_before_a_capture():
     assert dead() is None
 
 
+def test_graph_buffers_leave_the_whole_heap_alone():
+    """Only capture_graph pays for a full collection."""
+    import gc
+
+    from nanokv.packing import DecodeGraphBuffers
+
+    full = []
+
+    def watch(phase, info):
+        if phase == "start" and info["generation"] == 2:
+            full.append(info)
+
+    gc.disable()
+    gc.callbacks.append(watch)
+    try:
+        DecodeGraphBuffers.allocate("cpu", 2, 3)
+    finally:
+        gc.callbacks.remove(watch)
+        gc.enable()
+    assert not full
+
+
+@pytest.mark.parametrize("collector_on", [True, False])
+@pytest.mark.parametrize("fails", [False, True])
+def test_capture_graph_keeps_the_collector_out(monkeypatch, collector_on, fails):
+    """Dead cycles of any age are freed before the capture starts, the
+    collector is off until the last capture under way has ended, also when
+    one raises, and is then as it was."""
+    import gc
+    import weakref
+    from contextlib import contextmanager
+
+    from nanokv import packing
+
+    class Holder:
+        pass
+
+    old = Holder()
+    old.self = old
+    gc.collect()  # now of the oldest generation
+    dead = weakref.ref(old)
+    del old
+    seen = []
+
+    @contextmanager
+    def capture(graph, **options):
+        seen.append((graph, options, dead() is None, gc.isenabled()))
+        yield
+        seen.append(gc.isenabled())
+
+    monkeypatch.setattr(torch.cuda, "graph", capture)
+    (gc.enable if collector_on else gc.disable)()
+    try:
+        try:
+            with packing.capture_graph("outer", pool=3):
+                with packing.capture_graph("inner"):
+                    pass
+                assert not gc.isenabled()
+                if fails:
+                    raise RuntimeError("captured work failed")
+        except RuntimeError:
+            assert fails
+        assert gc.isenabled() == collector_on
+    finally:
+        gc.enable()
+    assert seen[:3] == [("outer", {"pool": 3}, True, False), ("inner", {}, True, False), False]
+    assert seen[3:] == ([] if fails else [False])
+
+
 def test_attention_calls_the_binding_leaves_to_the_general_path():
     """Host tensors, and calls any check of the general path looks into, are
     not taken by the binding's attention entries: they return None, and the
