@@ -301,7 +301,11 @@ def test_visibility_is_exact(backend, gpu_device, g, bs):
 
 def test_cache_over_4gib(backend, gpu_device):
     """Caches larger than 4 GiB, whose row byte offsets need more than 32
-    bits: the requests' blocks are moved to the top of each cache."""
+    bits: the requests' blocks are moved to the top of each cache.  Both the
+    launch that cuts its keys and the one of whole tiles."""
+    from nanokv import _lib
+    from nanokv.paged_kv import ops
+
     hkv, g, bs = 8, 2, 256
     q_lens, k_lens = [70, 5, 130], [300, 700, 130]
     dev, host = build_case(gpu_device, hkv, g, bs, q_lens, k_lens, seed=41, spare_blocks=0)
@@ -318,6 +322,18 @@ def test_cache_over_4gib(backend, gpu_device):
         out = backend.paged_attention_prefill(dev["q"], kc, vc, tables, dev["cu_q"], dev["cu_k"],
                                               scale)
         check_close(out, *reference(host, scale), "cache over 4 GiB")
+        # The launch above cuts its keys; without a workspace none are cut.
+        plan = backend.build_prefill_plan(dev["q"], kc, dev["cu_q"], dev["cu_k"])
+        library = _lib.load_library()
+        assert library.nkv_prefill_workspace_bytes(plan.shape[0], hkv, tables.shape[1] * bs) > 0
+        q, whole = dev["q"], torch.full_like(out, float("nan"))
+        _lib.check(library.nkv_paged_attention_prefill(
+            q.data_ptr(), q.stride(0), kc.data_ptr(), vc.data_ptr(), tables.data_ptr(),
+            tables.shape[1], dev["cu_q"].data_ptr(), dev["cu_k"].data_ptr(), plan.data_ptr(),
+            plan.shape[0], len(q_lens), hkv, hkv * g, 128, bs, big, scale,
+            ops.DTYPE_CODES[torch.bfloat16], whole.data_ptr(), whole.stride(0),
+            ops.current_stream_handle(gpu_device)), "prefill without a workspace")
+        check_close(whole, *reference(host, scale), "cache over 4 GiB, whole tiles")
     finally:
         del kc, vc
         torch.cuda.empty_cache()
@@ -433,6 +449,7 @@ def test_flash_varlen_contiguous_keys_matches_oracle(gpu_device):
     (1, 4, [33, 1], [2000, 513], "own"),
     (2, 3, [50, 60], [50, 60], "odd"),      # rows 8 bytes off 16: the paged path compacts them
     (2, 2, [40, 30], [90, 30], "short"),    # max_seqlen_k below a length: its last keys drop out
+    (2, 2, [300], [300], "far"),            # rows 16 MiB apart: byte offsets past 32 bits
 ])
 def test_flash_varlen_in_place_equals_the_paged_path(gpu_device, monkeypatch, hkv, g, q_lens, k_lens, layout):
     """Keys back to back, read where they lie: against the oracle, and equal
@@ -451,6 +468,9 @@ def test_flash_varlen_in_place_equals_the_paged_path(gpu_device, monkeypatch, hk
     elif layout == "kv":
         buf = torch.zeros((2, total, width + 8), dtype=torch.bfloat16, device=gpu_device)
         views = [buf[0, :, :width], buf[1, :, 8:]]
+    elif layout == "far":
+        buf = torch.empty((total, 1 << 23), dtype=torch.bfloat16, device=gpu_device)
+        views = [buf[:, :width], buf[:, -width:]]
     elif layout == "odd":
         buf = torch.zeros((2, total, width + 4), dtype=torch.bfloat16, device=gpu_device)
         views = [buf[0, :, :width], buf[1, :, 4:]]
