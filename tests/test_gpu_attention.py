@@ -586,7 +586,8 @@ def test_plan_from_lengths_equals_plan_from_offsets(backend, gpu_device, hkv, le
 @pytest.mark.parametrize("hkv,g,pad", [(8, 2, 0), (4, 7, 3), (2, 16, 1)])
 def test_host_binding_equals_the_general_path(backend, gpu_device, monkeypatch, hkv, g, pad):
     """Decode and prefill through the host binding and through the Python
-    checks: the same bits, new and given outputs, a strided q."""
+    checks: the same bits, new and given outputs, a strided q.  The binding
+    serves every call of the first pass."""
     from nanokv.paged_kv import hip_backend
 
     lens = [300, 1, 513, 40]
@@ -604,12 +605,70 @@ def test_host_binding_equals_the_general_path(backend, gpu_device, monkeypatch, 
                                                             cu_q, dev["cu"], 0.1, out=make()))
         return outs
 
+    served = []
+    for name in ("decode", "prefill"):
+        entry = getattr(hip_backend._HOST, name)
+        monkeypatch.setattr(hip_backend._HOST, name,
+                            lambda *a, entry=entry: served.append(entry(*a)) or served[-1])
     native = calls()
+    assert len(served) == len(native) and all(isinstance(out, torch.Tensor) for out in served)
     taken = []
     for name in ("decode", "prefill"):
         monkeypatch.setattr(hip_backend._HOST, name, lambda *a, name=name: taken.append(name))
     general = calls()
-    assert taken
+    assert len(taken) == len(general)
     for a, b in zip(native, general):
         assert torch.equal(a, b)
     check_close(native[0], reference(host, 0.1), "native decode")
+
+
+@pytest.mark.parametrize("what,error", [
+    ("index validation", None), ("no offsets", None), ("long plan", None),
+    ("short plan", "plan has"), ("strided table", "block_tables must be contiguous"),
+    ("int64 table", "int32"), ("wrong out shape", "out must match"), ("wrong out type", "one dtype"),
+    ("strided out heads", "out must match"), ("strided cache", "contiguous"), ("few offsets", "cu_seqlens_k"),
+])
+def test_calls_the_host_binding_passes_on(backend, gpu_device, monkeypatch, what, error):
+    """On the GPU: a planned decode call that is not as the kernels take it
+    gets None from the binding, and the general path serves or refuses it;
+    calls without offsets or with a longer plan are the binding's."""
+    from nanokv.paged_kv import hip_backend
+
+    lens = [300, 1, 513, 40]
+    dev, host, total = build_case(gpu_device, 8, 2, 16, lens, seed=3)
+    plan = backend.build_attention_plan(dev["kc"], dev["cu"], total)
+    q, kc, vc, tables, cu, out = dev["q"], dev["kc"], dev["vc"], dev["tables"], dev["cu"], None
+    pair = (plan[0], plan[1])  # not tied to the lengths it was built for
+    if what == "index validation":
+        monkeypatch.setenv("NANOVLLM_PAGED_KV_VALIDATE_INDICES", "1")
+    elif what == "long plan":
+        pair = (torch.cat([plan[0], torch.zeros_like(plan[0][:8])]), plan[1])
+    elif what == "short plan":
+        pair = (plan[0][:8], plan[1])
+    elif what == "strided table":
+        tables = torch.stack([tables, tables], dim=2)[:, :, 0]
+    elif what == "int64 table":
+        tables = tables.long()
+    elif what == "wrong out shape":
+        out = torch.zeros_like(q[:, :8])
+    elif what == "wrong out type":
+        out = torch.zeros_like(q, dtype=torch.float16)
+    elif what == "strided out heads":
+        out = torch.zeros((*q.shape[:2], 256), dtype=q.dtype, device=gpu_device)[:, :, :128]
+    elif what == "strided cache":
+        kc = torch.stack([kc, kc], dim=1)[:, 0]
+    elif what == "few offsets":
+        cu = cu[:-1]
+    binds = what in ("no offsets", "long plan")
+    got = hip_backend._HOST.decode(q, kc, vc, tables, None if what == "no offsets" else cu, *pair, total,
+                                   0.1, out, torch.cuda.current_stream().cuda_stream)
+    assert (got is not None) == binds
+    if error is None:
+        ref = reference(host, 0.1)
+        if binds:
+            check_close(got, ref, what)
+        check_close(backend.paged_attention_decode(q, kc, vc, tables, cu, total, 0.1, plan=pair, out=out),
+                    ref, what)
+    else:
+        with pytest.raises(ValueError, match=error):
+            backend.paged_attention_decode(q, kc, vc, tables, cu, total, 0.1, plan=pair, out=out)
