@@ -413,8 +413,9 @@ __device__ __forceinline__ void emit_partial(uint32_t* acc_out, f32x2* ml_out, f
 // short or few: one sequence of 5,003 rows is 7 entries, 56 workgroups of 8
 // kv heads, each walking 12 chunks per wave in a row.  Such a launch cuts
 // every entry in 2 where that makes at most kHalvesTarget workgroups (four
-// rounds of two per CU: 920 workgroups are 1.8 rounds, 1,840 halves pack
-// better, 12 layers of a 30-sequence step 782 -> 752 us), and further, up to
+// rounds of two per CU: the 95 entries of a 30-sequence step are 760
+// workgroups, 1.5 rounds, and 1,520 halves pack better, 12 layers of it 782
+// -> 752 us), and further, up to
 // 16, where that makes at most kPartsTarget (shorter parts cost more to start
 // than they balance: 23 sequences of 34k rows, 944 halves 31.5 us, 1,888
 // quarters 33.6).  The parts must fit the plan's capacity, which the partials
@@ -1166,13 +1167,15 @@ __global__ __launch_bounds__(kDecThreads) void attn_decode_range_kernel(
 // merge through LDS and the first divides once.
 // One batch after another costs about 0.8 us each, so a long context among
 // few sequences, cut into a hundred parts, took 14 us with one wave per pair
-// (8 sequences of 4 kv heads, 28 query heads): a pair gets 4 or 16 waves by
-// the average number of parts (reduce_waves).
+// (8 sequences of 4 kv heads, 28 query heads; 4.1 with 16): a pair gets 4 or
+// 16 waves by the parts per sequence that the host can tell (reduce_waves).
 constexpr int kReduceThreads = 4 * kWave;  // with one wave per pair: 4 pairs per workgroup
 constexpr int kReduceBatch = 8;            // parts in flight per lane
 
-// Waves per pair.  The parts of all sequences are about `parts` in all;
+// Waves per pair, for about `parts` parts in all sequences together;
 // contexts of unlike lengths give one sequence several times its share.
+// Thresholds of 16 and 4 parts a sequence instead of 8 and 2 made a captured
+// 12-layer step 773 us instead of 747.
 constexpr int reduce_waves(int64_t parts, int64_t num_seqs) {
   return parts > 8 * num_seqs ? 16 : parts > 2 * num_seqs ? 4 : 1;
 }
@@ -1515,7 +1518,12 @@ extern "C" int nkv_paged_attention_decode_total(
   }
   if (int rc = nkv_check_launch("nkv_paged_attention_decode (partials)")) return rc;
   const int4* const range_plan = entries ? nullptr : static_cast<const int4*>(plan);
-  // Parts of all sequences at most (long contexts of the entry split aside).
+  // The parts of all sequences, as far as the host can tell: the workers of
+  // a kv head (range split), or what entry_parts cuts short launches up to
+  // (entry split).  The entry split may have more: twice as many halves, and
+  // as many whole entries as long contexts make (at 8 kv heads 20 sequences
+  // of 32k rows, 43 parts each, are merged by 4 waves a pair, and 64 or more
+  // sequences of any length by one).
   const int64_t parts = entries ? kPartsTarget / num_kv_heads : workers_per_head(num_kv_heads);
   const int waves = reduce_waves(parts, num_seqs);
   const int64_t pairs = num_seqs * num_q_heads;

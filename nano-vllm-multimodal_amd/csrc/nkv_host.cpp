@@ -396,7 +396,7 @@ void bind(uintptr_t store_fn, uintptr_t gather_fn, uintptr_t last_error_fn) {
 }  // namespace
 
 PYBIND11_MODULE(_nkv_host, m) {
-  m.doc() = "Per-call host path of the nanokv hip backend's store and gather";
+  m.doc() = "Per-call host path of the nanokv hip backend's store, gather and attention";
   m.def("bind", &bind, "set the library entry points (nkv_store, nkv_gather, nkv_last_error)");
   m.def("bind_attention", &bind_attention, "set the library's attention entry points");
   m.def("decode", &decode, "planned decode attention; None when the general path has to look at it");

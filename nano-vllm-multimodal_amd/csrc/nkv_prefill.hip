@@ -311,19 +311,22 @@ __device__ __forceinline__ TileId tile_of(uint32_t id, int32_t num_kv_heads, int
 }
 
 // The key split.  A workgroup walks the keys of its query tile one 64-key
-// tile after another (about 1.3 us each), so a launch of few query tiles
+// tile after another (about 1.5 us each), so a launch of few query tiles
 // lasts as long as its longest one while most of the chip idles: 4 requests
-// of ~98 new tokens over 6k-12k cached ones are 64 workgroups (8 kv heads)
-// and took 262 us, 195 key tiles in a row on a quarter of the CUs.  Such a
-// launch cuts each tile's keys into pieces of at most C key tiles, one
-// workgroup each, whose fp32 partials (max, weight sum, output sums) a merge
-// kernel adds up: that case went to 57 us, one 40-token chunk over 14k
-// cached rows from 311 to 33 us.
+// of 391 new tokens over 7k-11k cached ones are 7 query tiles, 56 workgroups
+// (8 kv heads), and took 265 us, up to 169 key tiles in a row on a fifth of
+// the CUs.  Such a launch cuts each tile's keys into pieces of at most C key
+// tiles, one workgroup each, whose fp32 partials (max, weight sum, output
+// sums) a merge kernel adds up: that case went to 57-61 us (19 key tiles in
+// a row), one 40-token chunk over 14k cached rows from 311 to 33 us.
 // One kv head can have slots = 512 / Hkv workgroups resident at once (two
 // per CU).  With T key tiles in the whole plan, C = T / (slots - tiles)
 // makes at most T / C + tiles <= slots pieces, which start together; more
 // would leave a second, nearly empty round (with C = T / slots, 284
-// workgroups of 2 kv heads lost 5% instead).  A piece of fewer than
+// workgroups of 2 kv heads lost 5% instead).  The bound counts every tile's
+// remainder as a whole piece, so some slots stay free: 57 of 64 are taken
+// in the case above, 189 of 256 by one prompt of 1,511 tokens (2 kv heads).
+// A piece of fewer than
 // kSplitMinTiles key tiles costs more to start and merge than it saves (2,
 // 4 and 6 measure alike).
 #ifndef NKV_PF_SPLIT_MIN_TILES
@@ -346,8 +349,8 @@ __host__ __device__ constexpr int32_t split_slots(int64_t num_kv_heads) {
 // having more than max_keys of them: when it is one round of workgroups (cut
 // launches of two rounds and more lost 10-20%: 868 workgroups of 4 kv heads
 // took 80 us against 64) and some tile may see enough keys to pay for the
-// merge launch (about 4 us, three key tiles; 456 workgroups over at most 4
-// key tiles lost 7%).
+// merge launch (4 us with few pieces, three key tiles, and up to 15 with 56
+// pieces a tile; 456 workgroups over at most 4 key tiles lost 7%).
 constexpr bool uses_split(int64_t capacity, int64_t num_kv_heads, int64_t max_keys) {
   return num_kv_heads <= kSplitSlots && capacity * num_kv_heads <= kSplitSlots &&
          max_keys > int64_t{kSplitMinSeen} * kPfKeys;
@@ -436,10 +439,13 @@ __device__ __forceinline__ Piece find_piece(const int4* __restrict__ plan, int32
 // x 32 dims of one (tile, kv head); a lane holds the same row and dims as in
 // the attention kernel, so the row's weights need no exchange and every
 // access is 1 KiB.  Four pieces are in flight at once.  It waits for memory,
-// so more and smaller wavefronts help: with 64 dims each, one 40-token chunk
-// over 14k cached rows (56 pieces a tile) took 36.7 us instead of 32.7, the
-// other launches up to 1% more; 16 dims and eight pieces in flight were 2%
-// slower on those.  Blocks of padding rows are neither written nor read.
+// so more and smaller wavefronts help where a tile has many pieces: with 64
+// dims each, one 40-token chunk over 14k cached rows (56 pieces a tile) took
+// 35.6 us instead of 32.6, launches of 2 to 9 pieces a tile the same or up
+// to 2% more (391 tokens of 4 requests 54.2 instead of 53.6, one prompt of
+// 1,511 37.2 instead of 37.0; both in turn, four times).  16 dims and eight
+// pieces in flight took another 3 us off the first but cost those 2-5%.
+// Blocks of padding rows are neither written nor read.
 constexpr int kMergeBatch = 4;
 constexpr int kMergeWaves = 4;
 constexpr int kMergeParts = 4;  // wavefronts per 16 rows

@@ -159,8 +159,8 @@ def build(*, verbose: bool = False, output: Path | None = None,
 
 # ------------------------------------------------------------ host binding
 #
-# _nkv_host: the backend's per-call store / gather path in C++ (csrc/
-# nkv_host.cpp), a CPython extension compiled with g++ against torch's
+# _nkv_host: the backend's per-call store, gather and attention path in C++
+# (csrc/nkv_host.cpp), a CPython extension compiled with g++ against torch's
 # headers (it has no device code).  It is bound to the torch it was built
 # against, so torch's version is part of its fingerprint.
 
