@@ -250,6 +250,16 @@ at::Tensor output_for(const at::Tensor& q, const c10::optional<at::Tensor>& out)
 at::Tensor bytes_on(int64_t bytes, const at::Tensor& like) {
   return at::empty({bytes}, like.options().dtype(at::kByte));
 }
+// Room for the partials of a prefill launch that cuts its keys.  Undefined
+// where there is none to need, or to have: the launch then cuts nothing.
+at::Tensor partials_on(int64_t bytes, const at::Tensor& like) {
+  if (bytes <= 0) return {};
+  try {
+    return bytes_on(bytes, like);
+  } catch (const c10::OutOfMemoryError&) {
+    return {};
+  }
+}
 void* data_or_null(const at::Tensor& t) { return t.size(0) > 0 ? t.data_ptr() : nullptr; }
 
 // The offsets are only checked (the plan holds what the kernels need);
@@ -326,13 +336,13 @@ py::object prefill(const at::Tensor& q, const at::Tensor& key_cache, const at::T
   const at::Tensor plan = plan_in.has_value() ? *plan_in : prefill_plan(q, kv_heads, cu_q, cu_k, stream);
   if (!plan.defined()) return py::none();
   const int64_t need = g_prefill_workspace(plan.size(0), kv_heads, tables.size(1) * key_cache.size(1));
-  const at::Tensor workspace = need > 0 ? bytes_on(need, q) : at::Tensor();
+  const at::Tensor workspace = partials_on(need, q);
   check_status(g_prefill(q.data_ptr(), q.stride(0), key_cache.data_ptr(), value_cache.data_ptr(),
                          tables.data_ptr<int32_t>(), tables.size(1), cu_q.data_ptr<int32_t>(),
                          cu_k.data_ptr<int32_t>(), data_or_null(plan), plan.size(0), seqs, kv_heads,
                          q.size(1), kDim, key_cache.size(1), key_cache.size(0),
                          static_cast<float>(scale), dtype_code(type), out.data_ptr(), out.stride(0),
-                         need > 0 ? workspace.data_ptr() : nullptr, need,
+                         workspace.defined() ? workspace.data_ptr() : nullptr, need,
                          reinterpret_cast<void*>(stream)),
                "nanovllm_paged_kv::paged_attention_prefill");
   return py::cast(out);
@@ -363,12 +373,12 @@ py::object varlen(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
   const at::Tensor out = at::empty_like(q);
   const int64_t longest = std::max<int64_t>(max_seqlen_k, 1);
   const int64_t need = g_prefill_workspace(plan.size(0), kv_heads, longest);
-  const at::Tensor workspace = need > 0 ? bytes_on(need, q) : at::Tensor();
+  const at::Tensor workspace = partials_on(need, q);
   check_status(g_varlen(q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(),
                         v.stride(0), k.size(0), longest, cu_q.data_ptr<int32_t>(),
                         cu_k.data_ptr<int32_t>(), plan.data_ptr(), plan.size(0), seqs, kv_heads,
                         q.size(1), kDim, static_cast<float>(scale), dtype_code(type), out.data_ptr(),
-                        out.stride(0), need > 0 ? workspace.data_ptr() : nullptr, need,
+                        out.stride(0), workspace.defined() ? workspace.data_ptr() : nullptr, need,
                         reinterpret_cast<void*>(stream)),
                "nanovllm_paged_kv::varlen_attention_prefill");
   return py::cast(out);

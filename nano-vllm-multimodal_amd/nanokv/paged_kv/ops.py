@@ -530,17 +530,23 @@ def _paged_attention_prefill_impl(q, key_cache, value_cache, block_tables, cu_se
         if plan.shape[0] < need:
             raise ValueError(f"prefill plan has {plan.shape[0]} entries, these queries need {need}: "
                              "build it with build_prefill_plan for the same q and cu_seqlens")
-    # Partials of a launch that cuts its keys (none for one that fills the chip).
+    # Partials of a launch that cuts its keys (none for one that fills the
+    # chip); where they do not fit, the launch cuts nothing.
     nbytes = int(library.nkv_prefill_workspace_bytes(
         plan.shape[0], num_kv_heads, block_tables.shape[1] * block_size))
-    workspace = torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes else None
+    workspace = None
+    if nbytes:
+        try:
+            workspace = torch.empty(nbytes, dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError:
+            pass
     status = library.nkv_paged_attention_prefill_split(
         q.data_ptr(), q.stride(0), key_cache.data_ptr(), value_cache.data_ptr(),
         block_tables.data_ptr(), block_tables.shape[1], cu_seqlens_q.data_ptr(),
         cu_seqlens_k.data_ptr(), plan.data_ptr() if plan.shape[0] else None, plan.shape[0],
         num_seqs, num_kv_heads, q.shape[1], head_dim, block_size, num_blocks, float(scale),
         DTYPE_CODES[q.dtype], out.data_ptr(), out.stride(0),
-        workspace.data_ptr() if nbytes else None, nbytes, _stream(device),
+        None if workspace is None else workspace.data_ptr(), nbytes, _stream(device),
     )
     _lib.check(status, "nanovllm_paged_kv::paged_attention_prefill")
 

@@ -12,6 +12,7 @@ exactly by test_visibility_is_exact (uniform weights, indicator values).
 """
 from __future__ import annotations
 
+import contextlib
 import math
 
 import numpy as np
@@ -623,3 +624,46 @@ def test_flash_dropins_reject_what_they_do_not_compute(gpu_device):
         flash_attn_with_kvcache(dev["q"][:1].unsqueeze(1), dev["kc"], dev["vc"],
                                 cache_seqlens=dev["cu_k"][1:], block_table=dev["tables"],
                                 causal=True, rotary_cos=None)
+
+
+@contextlib.contextmanager
+def no_more_memory(device):
+    """torch's allocator at its limit: what is not cached yet is refused."""
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(device).total_memory
+    torch.cuda.set_per_process_memory_fraction(torch.cuda.memory_reserved(device) / total, device)
+    try:
+        yield
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, device)
+
+
+@pytest.mark.parametrize("general", [False, True])
+def test_short_launches_need_no_memory(backend, gpu_device, monkeypatch, general):
+    """At the memory limit, where the partials of a cut launch do not fit,
+    the launch cuts nothing and the call is served as without a workspace."""
+    from nanokv import _lib
+    from nanokv.paged_kv import hip_backend, ops
+
+    if general:
+        monkeypatch.setattr(hip_backend._HOST, "prefill", lambda *args: None)
+    hkv, g, bs = 8, 2, 256
+    dev, host = build_case(gpu_device, hkv, g, bs, [98, 65], [3001, 2113], seed=11)
+    scale = 1.0 / math.sqrt(128)
+    q, kc = dev["q"], dev["kc"]
+    plan = backend.build_prefill_plan(q, kc, dev["cu_q"], dev["cu_k"])
+    out = torch.full_like(q.contiguous(), float("nan"))
+    whole = torch.full_like(out, float("nan"))
+    _lib.check(_lib.load_library().nkv_paged_attention_prefill(
+        q.data_ptr(), q.stride(0), kc.data_ptr(), dev["vc"].data_ptr(), dev["tables"].data_ptr(),
+        dev["tables"].shape[1], dev["cu_q"].data_ptr(), dev["cu_k"].data_ptr(), plan.data_ptr(),
+        plan.shape[0], 2, hkv, hkv * g, 128, bs, kc.shape[0], scale,
+        ops.DTYPE_CODES[torch.bfloat16], whole.data_ptr(), whole.stride(0),
+        ops.current_stream_handle(gpu_device)), "prefill without a workspace")
+    with no_more_memory(gpu_device):
+        run(backend, dev, scale, plan=plan, out=out)
+    assert torch.equal(out, whole)
+    run(backend, dev, scale, plan=plan, out=out)  # with memory again: cut, and close
+    assert not torch.equal(out, whole)
+    check_close(out, *reference(host, scale), "after the limit")
