@@ -264,6 +264,20 @@ void* data_or_null(const at::Tensor& t) { return t.size(0) > 0 ? t.data_ptr() : 
 
 // The offsets are only checked (the plan holds what the kernels need);
 // callers that built the plan from the lengths have none.
+// The checked part of a call, which allocates and launches and may wait for
+// either, without the interpreter lock, as in torch's own calls and through
+// ctypes; None where it gives no tensor.
+template <typename Launch>
+py::object run_unlocked(Launch&& launch) {
+  at::Tensor out;
+  {
+    py::gil_scoped_release unlocked;
+    out = launch();
+  }
+  if (!out.defined()) return py::none();
+  return py::cast(out);
+}
+
 py::object decode(const at::Tensor& q, const at::Tensor& key_cache, const at::Tensor& value_cache,
                   const at::Tensor& tables, const c10::optional<at::Tensor>& cu_seqlens_k,
                   const at::Tensor& plan, const at::Tensor& first_part, int64_t total_tokens,
@@ -285,19 +299,21 @@ py::object decode(const at::Tensor& q, const at::Tensor& key_cache, const at::Te
       plan.size(0) < g_decode_capacity(total_tokens, seqs, key_cache.size(1))) {
     return py::none();
   }
-  const at::Tensor out = output_for(q, out_in);
-  if (!out.defined()) return py::none();
-  const int64_t capacity = plan.size(0);
-  const int64_t need = std::max<int64_t>(g_decode_workspace(capacity, q.size(1), kDim), 16);
-  const at::Tensor workspace = bytes_on(need, q);
-  check_status(g_decode(q.data_ptr(), q.stride(0), key_cache.data_ptr(), value_cache.data_ptr(),
-                        tables.data_ptr<int32_t>(), tables.size(1), data_or_null(plan), capacity,
-                        first_part.data_ptr<int32_t>(), seqs, key_cache.size(2), q.size(1), kDim,
-                        key_cache.size(1), key_cache.size(0), static_cast<float>(scale),
-                        dtype_code(type), workspace.data_ptr(), need, out.data_ptr(), out.stride(0),
-                        total_tokens, reinterpret_cast<void*>(stream)),
-               "nanovllm_paged_kv::paged_attention_decode");
-  return py::cast(out);
+  return run_unlocked([&]() -> at::Tensor {
+    const at::Tensor out = output_for(q, out_in);
+    if (!out.defined()) return {};
+    const int64_t capacity = plan.size(0);
+    const int64_t need = std::max<int64_t>(g_decode_workspace(capacity, q.size(1), kDim), 16);
+    const at::Tensor workspace = bytes_on(need, q);
+    check_status(g_decode(q.data_ptr(), q.stride(0), key_cache.data_ptr(), value_cache.data_ptr(),
+                          tables.data_ptr<int32_t>(), tables.size(1), data_or_null(plan), capacity,
+                          first_part.data_ptr<int32_t>(), seqs, key_cache.size(2), q.size(1), kDim,
+                          key_cache.size(1), key_cache.size(0), static_cast<float>(scale),
+                          dtype_code(type), workspace.data_ptr(), need, out.data_ptr(), out.stride(0),
+                          total_tokens, reinterpret_cast<void*>(stream)),
+                 "nanovllm_paged_kv::paged_attention_decode");
+    return out;
+  });
 }
 
 // A prefill plan for these offsets, or undefined where the head layout has none.
@@ -331,21 +347,23 @@ py::object prefill(const at::Tensor& q, const at::Tensor& key_cache, const at::T
        plan_in->size(0) < g_prefill_capacity(q.size(0), seqs, q.size(1) / kv_heads))) {
     return py::none();
   }
-  const at::Tensor out = output_for(q, out_in);
-  if (!out.defined()) return py::none();
-  const at::Tensor plan = plan_in.has_value() ? *plan_in : prefill_plan(q, kv_heads, cu_q, cu_k, stream);
-  if (!plan.defined()) return py::none();
-  const int64_t need = g_prefill_workspace(plan.size(0), kv_heads, tables.size(1) * key_cache.size(1));
-  const at::Tensor workspace = partials_on(need, q);
-  check_status(g_prefill(q.data_ptr(), q.stride(0), key_cache.data_ptr(), value_cache.data_ptr(),
-                         tables.data_ptr<int32_t>(), tables.size(1), cu_q.data_ptr<int32_t>(),
-                         cu_k.data_ptr<int32_t>(), data_or_null(plan), plan.size(0), seqs, kv_heads,
-                         q.size(1), kDim, key_cache.size(1), key_cache.size(0),
-                         static_cast<float>(scale), dtype_code(type), out.data_ptr(), out.stride(0),
-                         workspace.defined() ? workspace.data_ptr() : nullptr, need,
-                         reinterpret_cast<void*>(stream)),
-               "nanovllm_paged_kv::paged_attention_prefill");
-  return py::cast(out);
+  return run_unlocked([&]() -> at::Tensor {
+    const at::Tensor out = output_for(q, out_in);
+    if (!out.defined()) return {};
+    const at::Tensor plan = plan_in.has_value() ? *plan_in : prefill_plan(q, kv_heads, cu_q, cu_k, stream);
+    if (!plan.defined()) return {};
+    const int64_t need = g_prefill_workspace(plan.size(0), kv_heads, tables.size(1) * key_cache.size(1));
+    const at::Tensor workspace = partials_on(need, q);
+    check_status(g_prefill(q.data_ptr(), q.stride(0), key_cache.data_ptr(), value_cache.data_ptr(),
+                           tables.data_ptr<int32_t>(), tables.size(1), cu_q.data_ptr<int32_t>(),
+                           cu_k.data_ptr<int32_t>(), data_or_null(plan), plan.size(0), seqs, kv_heads,
+                           q.size(1), kDim, key_cache.size(1), key_cache.size(0),
+                           static_cast<float>(scale), dtype_code(type), out.data_ptr(), out.stride(0),
+                           workspace.defined() ? workspace.data_ptr() : nullptr, need,
+                           reinterpret_cast<void*>(stream)),
+                 "nanovllm_paged_kv::paged_attention_prefill");
+    return out;
+  });
 }
 
 // Keys and values back to back, read where they lie: rows of [kv_heads, 128]
@@ -367,21 +385,23 @@ py::object varlen(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v,
       return py::none();
     }
   }
-  const int64_t seqs = cu_q.size(0) - 1, kv_heads = k.size(1);
-  const at::Tensor plan = prefill_plan(q, kv_heads, cu_q, cu_k, stream);
-  if (!plan.defined()) return py::none();
-  const at::Tensor out = at::empty_like(q);
-  const int64_t longest = std::max<int64_t>(max_seqlen_k, 1);
-  const int64_t need = g_prefill_workspace(plan.size(0), kv_heads, longest);
-  const at::Tensor workspace = partials_on(need, q);
-  check_status(g_varlen(q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(),
-                        v.stride(0), k.size(0), longest, cu_q.data_ptr<int32_t>(),
-                        cu_k.data_ptr<int32_t>(), plan.data_ptr(), plan.size(0), seqs, kv_heads,
-                        q.size(1), kDim, static_cast<float>(scale), dtype_code(type), out.data_ptr(),
-                        out.stride(0), workspace.defined() ? workspace.data_ptr() : nullptr, need,
-                        reinterpret_cast<void*>(stream)),
-               "nanovllm_paged_kv::varlen_attention_prefill");
-  return py::cast(out);
+  return run_unlocked([&]() -> at::Tensor {
+    const int64_t seqs = cu_q.size(0) - 1, kv_heads = k.size(1);
+    const at::Tensor plan = prefill_plan(q, kv_heads, cu_q, cu_k, stream);
+    if (!plan.defined()) return {};
+    const at::Tensor out = at::empty_like(q);
+    const int64_t longest = std::max<int64_t>(max_seqlen_k, 1);
+    const int64_t need = g_prefill_workspace(plan.size(0), kv_heads, longest);
+    const at::Tensor workspace = partials_on(need, q);
+    check_status(g_varlen(q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0), v.data_ptr(),
+                          v.stride(0), k.size(0), longest, cu_q.data_ptr<int32_t>(),
+                          cu_k.data_ptr<int32_t>(), plan.data_ptr(), plan.size(0), seqs, kv_heads,
+                          q.size(1), kDim, static_cast<float>(scale), dtype_code(type), out.data_ptr(),
+                          out.stride(0), workspace.defined() ? workspace.data_ptr() : nullptr, need,
+                          reinterpret_cast<void*>(stream)),
+                 "nanovllm_paged_kv::varlen_attention_prefill");
+    return out;
+  });
 }
 
 void bind_attention(uintptr_t decode_capacity, uintptr_t decode_workspace, uintptr_t decode_fn,

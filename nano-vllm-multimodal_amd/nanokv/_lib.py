@@ -269,8 +269,16 @@ _HOST_LOCK = Lock()
 _HOST = None
 
 
+# The host binding's attention entry points, in bind_attention's order.
+HOST_ATTENTION_ENTRIES = (
+    "nkv_attention_plan_capacity", "nkv_attention_workspace_bytes", "nkv_paged_attention_decode_total",
+    "nkv_prefill_plan_capacity", "nkv_build_prefill_plan", "nkv_prefill_workspace_bytes",
+    "nkv_paged_attention_prefill_split", "nkv_varlen_attention_prefill",
+)
+
+
 def load_host():
-    """The C++ host binding of the backend's per-call store and gather
+    """The C++ host binding of the backend's store, gather and attention calls
     (``nanokv._nkv_host``), bound to the loaded library's entry points.  A
     missing or stale binding raises RuntimeError: there is no slower path
     to fall back to silently."""
@@ -301,11 +309,7 @@ def load_host():
                 return ctypes.cast(getattr(library, name), ctypes.c_void_p).value
 
             module.bind(address("nkv_store"), address("nkv_gather"), address("nkv_last_error"))
-            module.bind_attention(*(address(name) for name in (
-                "nkv_attention_plan_capacity", "nkv_attention_workspace_bytes",
-                "nkv_paged_attention_decode_total", "nkv_prefill_plan_capacity",
-                "nkv_build_prefill_plan", "nkv_prefill_workspace_bytes",
-                "nkv_paged_attention_prefill_split", "nkv_varlen_attention_prefill")))
+            module.bind_attention(*map(address, HOST_ATTENTION_ENTRIES))
             _HOST = module
     return _HOST
 

@@ -672,3 +672,58 @@ def test_calls_the_host_binding_passes_on(backend, gpu_device, monkeypatch, what
     else:
         with pytest.raises(ValueError, match=error):
             backend.paged_attention_decode(q, kc, vc, tables, cu, total, 0.1, plan=pair, out=out)
+
+
+def test_other_threads_run_during_a_binding_call(backend, gpu_device, tmp_path):
+    """A launch may wait, for a full queue say: the process's other Python
+    threads go on meanwhile, as they do in torch's calls and ctypes'.  The
+    library's launches are replaced by a function that sleeps."""
+    import ctypes
+    import subprocess
+    import threading
+    import time
+
+    from nanokv import _lib
+
+    source, slow = tmp_path / "slow.c", tmp_path / "slow.so"
+    source.write_text("#include <unistd.h>\nint slow(void) { usleep(200000); return 0; }\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", str(source), "-o", str(slow)], check=True)
+    sleeps = ctypes.cast(ctypes.CDLL(str(slow)).slow, ctypes.c_void_p).value
+    library, host = _lib.load_library(), _lib.load_host()
+    entries = [ctypes.cast(getattr(library, name), ctypes.c_void_p).value
+               for name in _lib.HOST_ATTENTION_ENTRIES]
+    launches = ("decode_total", "prefill_split", "attention_prefill")
+    dev, _, total = build_case(gpu_device, 8, 2, 16, [40, 7], seed=1)
+    plan = backend.build_attention_plan(dev["kc"], dev["cu"], total)
+    cu_q = torch.arange(3, dtype=torch.int32, device=gpu_device)
+    rows = torch.zeros((total, 8, 128), dtype=torch.bfloat16, device=gpu_device)
+    calls = {
+        "decode": lambda: backend.paged_attention_decode(dev["q"], dev["kc"], dev["vc"], dev["tables"],
+                                                         dev["cu"], total, 0.1, plan=plan),
+        "prefill": lambda: backend.paged_attention_prefill(dev["q"], dev["kc"], dev["vc"], dev["tables"],
+                                                           cu_q, dev["cu"], 0.1),
+        "varlen": lambda: backend.varlen_attention_prefill(dev["q"], rows, rows, cu_q, dev["cu"], 40, 0.1),
+    }
+    for call in calls.values():
+        call()
+    ticks, stop = [], threading.Event()
+
+    def tick():
+        while not stop.wait(0.005):
+            ticks.append(time.perf_counter())
+
+    thread = threading.Thread(target=tick)
+    thread.start()
+    try:
+        host.bind_attention(*(sleeps if name.endswith(launches) else entry
+                              for name, entry in zip(_lib.HOST_ATTENTION_ENTRIES, entries)))
+        for name, call in calls.items():
+            began = time.perf_counter()
+            call()
+            ended = time.perf_counter()
+            assert ended - began > 0.19, name
+            assert sum(began < t < ended for t in ticks) >= 5, name
+    finally:
+        host.bind_attention(*entries)
+        stop.set()
+        thread.join()
